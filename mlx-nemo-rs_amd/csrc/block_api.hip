@@ -94,7 +94,10 @@ int32_t prepare_ffn(mhsa_ffn* f) {
     f->dev[i].sb = f->lin[i].quantized ? reinterpret_cast<const float*>(base + sboff[i]) : nullptr;
     f->dev[i].bias = f->lin[i].bias.empty() ? nullptr : reinterpret_cast<const float*>(base + boff[i]);
     f->dev32[i] = f->dev[i];
-    if (!f->lin[i].quantized && bf) f->dev32[i].w = base + w32off[i];
+    if (!f->lin[i].quantized && bf) {
+      f->dev32[i].w = base + w32off[i];
+      f->dev32[i].w16 = f->dev[i].w;
+    }
   }
   f->dirty = false;
   return MHSA_OK;
@@ -109,6 +112,7 @@ mhsa::GemmParams ffn_gemm(mhsa_ffn* f, int i, DType act, const void* A, int rows
   p.A = A;
   p.lda = ffn_in(f, i);
   p.W = d.w;
+  p.W16 = d.w16;
   p.sb = d.sb;
   p.bias = d.bias;
   p.C = C;
@@ -429,7 +433,10 @@ int32_t prepare_conv(mhsa_conv* m) {
     d.sb = d.quantized ? reinterpret_cast<const float*>(base + sboff[i]) : nullptr;
     d.bias = m->lin[i].bias.empty() ? nullptr : reinterpret_cast<const float*>(base + boff[i]);
     m->dev32[i] = d;
-    if (!d.quantized && bf) m->dev32[i].w = base + w32off[i];
+    if (!d.quantized && bf) {
+      m->dev32[i].w = base + w32off[i];
+      m->dev32[i].w16 = d.w;
+    }
   }
   m->taps = reinterpret_cast<const float*>(base + toff);
   m->taps_bias = m->dw_b.empty() ? nullptr : reinterpret_cast<const float*>(base + tboff);
@@ -446,6 +453,7 @@ int32_t conv_pointwise(mhsa_conv* m, int i, DType act, const void* A, int rows, 
   p.A = A;
   p.lda = m->D;
   p.W = d.w;
+  p.W16 = d.w16;
   p.sb = d.sb;
   p.bias = d.bias;
   p.C = C;

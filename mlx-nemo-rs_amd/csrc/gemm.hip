@@ -9,6 +9,9 @@
 //  * gemm_tile_kernel: bf16 projections with enough rows to fill the GPU
 //    (128x128, 192x128, 192x192, 192x256 or 256x256 tiles on 4 waves, direct-to-LDS operand
 //    streams, LDS-staged epilogue; described at its definition).
+//  * gemm_f32_tile_kernel: fp32 activations (with fp32, bf16 or u8 weights)
+//    on the bf16 matrix cores, each fp32 value as three bf16 ones
+//    (gemm_f32_tile.hpp).
 //  * gemm_kpar_kernel: fp32 projections of few rows (the streaming chunk,
 //    one short utterance): persistent workgroups over 32 x 32 tiles, each
 //    tile's contraction split over the K / 64 waves of a workgroup and summed
@@ -16,10 +19,10 @@
 //  * gemm_split_kernel + gemm_reduce: bf16 projections of few rows (the
 //    position table of a short utterance): K split over workgroups, the
 //    partial sums added in split order by a second kernel.
-//  * gemm_kernel: everything else (large fp32 problems; bf16 shapes the tile
-//    kernel does not take): BM x BN tiles on NWM x NWN waves, one 128-byte
-//    K step per LDS stage, double-buffered with a 16-byte row pad; an
-//    optional deterministic K split with gemm_reduce.
+//  * gemm_kernel: everything else (shapes and alignments the others do not
+//    take): BM x BN tiles on NWM x NWN waves, one 128-byte K step per LDS
+//    stage, double-buffered with a 16-byte row pad; an optional deterministic
+//    K split with gemm_reduce.
 //
 // With seg_T > 0 the M tiles are laid out per utterance (rows b*seg_T ..
 // (b+1)*seg_T, never straddling two), so the V projection can be written
@@ -38,6 +41,7 @@ constexpr int ROWB = 128;         // bytes of one tile row per K step
 constexpr int PITCH = ROWB + 16;  // LDS row pitch (bytes)
 
 #include "gemm_tile.hpp"
+#include "gemm_f32_tile.hpp"
 
 template <typename T, bool QUANT, int BN, int NT>
 struct BLoad;
@@ -773,31 +777,93 @@ hipError_t launch(const GemmParams& p, int splits, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <typename T, bool QUANT>
-hipError_t dispatch(const GemmParams& p, hipStream_t s) {
+// K splits of 64x64 tiles of the general kernel, until ~512 workgroups.
+template <typename T>
+int small_splits(const GemmParams& p) {
   const int bk = ROWB / (int)sizeof(T);
-  if constexpr (sizeof(T) == 4) {
-    if (p.C2 || p.acopy) return launch_kpar<QUANT>(p, s);  // (validated by gemm())
+  const int64_t tiles = m_tiles<64>(p) * (p.N / 64);
+  int splits = 1;
+  while (p.partial && tiles * splits * 2 <= 512 && p.K % (splits * 2 * bk) == 0 && p.K / (splits * 2) >= 2 * bk &&
+         (int64_t)splits * 2 * p.M * p.N <= p.partial_elems)
+    splits *= 2;
+  return splits;
+}
+
+// The fp32 tile kernel's operands: 16-byte rows addressable by 32-bit buffer
+// offsets.
+bool f32_tile_ok(const GemmParams& p) {
+  auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  if (p.vt || p.seg_T || p.K % 64 || p.N % 64 || p.lda % 4 || p.ldc % 4 || (p.R && p.ldr % 4)) return false;
+  if (!a16(p.A) || !a16(p.W) || !a16(p.W16) || !a16(p.C) || !a16(p.R) || !a16(p.bias) || !a16(p.sb)) return false;
+  if (p.C2 && (!a16(p.C2) || p.ldc2 % 4 || p.c2_col0 % 4)) return false;
+  return (int64_t)p.M * p.lda * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31);
+}
+
+template <int BM, int BN, int MW, int NW, int KW, int WK>
+hipError_t launch_f32_tile(const GemmParams& p, int splits, hipStream_t s) {
+  const int64_t items = (int64_t)((p.M + BM - 1) / BM) * (p.N / BN) * splits;
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN, MW, NW, KW, WK, 2>), dim3((unsigned)((items + 7) / 8 * 8)),
+                     dim3(64 * MW * NW * KW), 0, s, p, splits);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || splits == 1) return e;
+  hipLaunchKernelGGL((gemm_f32_reduce_kernel<WK>), dim3((unsigned)(((int64_t)p.M * p.N / 4 + 255) / 256)), dim3(256), 0,
+                     s, p, splits);
+  return hipGetLastError();
+}
+
+// fp32 activations. The K-parallel kernel has the shorter chain (16 waves
+// share a tile's contraction, 16x16 tiles), the tile kernel the higher rate,
+// so the line is where the K-parallel kernel's work per CU grows past one
+// short tile: 128 tiles of 32x32, 256 where its MFMAs are the same work as
+// the tile kernel's (fp32 weights: three times the products of bf16 ones) or
+// its contraction is short. Measured, us, K-parallel against tile kernel,
+// K = 1024: fp32 weights 224 x 1024 9.9 / 11.5, 56 x 4096 9.7 / 11.3, 300 x
+// 1024 14.0 / 11.8; u8 112 x 1024 9.9 / 11.5, 56 x 4096 13.5 / 11.9; bf16 112
+// x 1024 7.0 / 8.0, 56 x 4096 9.7 / 8.0; u8 125 x 2048 at K = 512 7.1 / 7.9.
+//
+// Tile: the large one (64 x 128 for bf16 weights, 64 x 64 else) from 512
+// tiles, two per CU, on; 32 x 64 below (1500 x 4096 x 1024: bf16 44 / 54,
+// fp32 85 / 102, u8 88 / 109 us; 1500 x 1024 x 1024: bf16 18.2 / 15.5, fp32
+// 28.3 / 27.4, u8 28.8 / 27.9; 450 x 4096 fp32 30 / 34).
+// A contraction past 1024 is split while the tiles stay under three per CU
+// (K = 4096, N = 1024, fp32 weights: 14 rows 32 -> 10.6 in eight, 224 rows
+// 35 -> 22.6 in four, 700 rows 59 -> 48 in two, the sum pass included).
+template <int WK>
+hipError_t dispatch_f32(const GemmParams& p, hipStream_t s) {
+  if (kpar_ok<float>(p)) {
+    const int64_t t32 = (int64_t)((p.M + 31) / 32) * (p.N / 32);
+    const bool wide = WK == kWF32 || (WK == kWU8 && p.K <= 512);
+    if (t32 <= (wide ? 256 : 128) || !f32_tile_ok(p)) return launch_kpar<WK == kWU8>(p, s);
   }
-  if constexpr (sizeof(T) == 2) {
-    hipError_t err;
-    if (dispatch_tile<QUANT>(p, s, err)) return err;
+  if (f32_tile_ok(p)) {
+    constexpr int BN = WK == kWBF16 ? 128 : 64, MW = WK == kWBF16 ? 2 : 1, KW = WK == kWBF16 ? 2 : 4;
+    if (p.N % BN == 0 && (int64_t)((p.M + 63) / 64) * (p.N / BN) >= 512)
+      return launch_f32_tile<64, BN, MW, 1, KW, WK>(p, 1, s);
+    const int64_t tiles = (int64_t)((p.M + 31) / 32) * (p.N / 64);
+    int splits = 1;
+    while (p.K > 1024 && p.partial && splits < 8 && tiles * splits * 2 <= 768 && p.K / 64 >= splits * 2 * 4 &&
+           (int64_t)splits * 2 * p.M * p.N <= p.partial_elems)
+      splits *= 2;
+    return launch_f32_tile<32, 64, 1, 1, 4, WK>(p, splits, s);
   }
+  // operands that are not in 16-byte rows
+  return launch<float, WK == kWU8, 64, 64, 2, 2>(p, small_splits<float>(p), s);
+}
+
+template <bool QUANT>
+hipError_t dispatch_bf16(const GemmParams& p, hipStream_t s) {
+  using T = bf16;
+  hipError_t err;
+  if (dispatch_tile<QUANT>(p, s, err)) return err;
   // 256x256 (8 waves) when it still fills the GPU about twice over: it
   // halves the LDS and L2 traffic per flop of 128x128 (measured 1.15x on
-  // M = 15000, N = 3072); bf16 only (fp32 accumulators would not fit).
-  if (sizeof(T) == 2 && p.N % 256 == 0 && m_tiles<256>(p) * (p.N / 256) >= 512 &&
+  // M = 15000, N = 3072).
+  if (p.N % 256 == 0 && m_tiles<256>(p) * (p.N / 256) >= 512 &&
       (!p.vt || (p.vt_Tpad % 256 == 0 && p.vt_col0 % 256 == 0)))
     return launch<T, QUANT, 256, 256, 4, 2>(p, 1, s);
   if (m_tiles<128>(p) * (p.N / 128) >= 384 && p.N % 128 == 0) return launch<T, QUANT, 128, 128, 2, 2>(p, 1, s);
   if (p.vt) return launch<T, QUANT, 128, 128, 2, 2>(p, 1, s);  // V^T epilogue needs whole 128-row tiles
-  // few rows of fp32: K-parallel workgroups, no second kernel (for bf16 the
-  // position table of a short utterance measured the same as split-K: 13.4
-  // against 12.6 us at 749 x 1024 x 1024, so bf16 keeps split-K); the split
-  // output and row copy only exist there
-  if constexpr (sizeof(T) == 4) {
-    if (kpar_ok<T>(p)) return launch_kpar<QUANT>(p, s);
-  }
+  // few rows (the position table of a short utterance)
   if (const int splits = split_count<T>(p)) {
     const int64_t tiles = (int64_t)((p.M + 63) / 64) * (p.N / 64);
     hipLaunchKernelGGL((gemm_split_kernel<T, QUANT>), dim3((unsigned)(tiles * splits)), dim3(256), 0, s, p, splits);
@@ -809,19 +875,13 @@ hipError_t dispatch(const GemmParams& p, hipStream_t s) {
     hipLaunchKernelGGL(gemm_reduce<T>, dim3(blocks), dim3(256), 0, s, p, splits);
     return hipGetLastError();
   }
-  // Small problem: 64x64 tiles, and K splits until ~512 workgroups.
-  const int64_t tiles = m_tiles<64>(p) * (p.N / 64);
-  int splits = 1;
-  while (p.partial && tiles * splits * 2 <= 512 && p.K % (splits * 2 * bk) == 0 && p.K / (splits * 2) >= 2 * bk &&
-         (int64_t)splits * 2 * p.M * p.N <= p.partial_elems)
-    splits *= 2;
-  return launch<T, QUANT, 64, 64, 2, 2>(p, splits, s);
+  return launch<T, QUANT, 64, 64, 2, 2>(p, small_splits<T>(p), s);
 }
 
 }  // namespace
 
 bool gemm_split_fused_ok(DType dt, const GemmParams& p) {
-  if (dt != kF32 || p.vt || !kpar_ok<float>(p)) return false;
+  if (dt != kF32 || p.vt || (!kpar_ok<float>(p) && !f32_tile_ok(p))) return false;
   if (p.C2 && (p.c2_col0 <= 0 || p.c2_col0 >= p.N || p.c2_col0 % 32 || p.ldc2 < p.N - p.c2_col0)) return false;
   if (p.acopy && (p.acopy_ld < p.K || (p.acopy_ld % 4) || (reinterpret_cast<uintptr_t>(p.acopy) & 15))) return false;
   return true;
@@ -905,8 +965,9 @@ hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmP
 hipError_t gemm(DType dt, bool quantized, const GemmParams& p, hipStream_t s) {
   if (p.M <= 0) return hipSuccess;
   if (hipError_t e = gemm_check(dt, quantized, p)) return e;
-  if (dt == kF32) return quantized ? dispatch<float, true>(p, s) : dispatch<float, false>(p, s);
-  return quantized ? dispatch<bf16, true>(p, s) : dispatch<bf16, false>(p, s);
+  if (dt == kF32)
+    return quantized ? dispatch_f32<kWU8>(p, s) : p.W16 ? dispatch_f32<kWBF16>(p, s) : dispatch_f32<kWF32>(p, s);
+  return quantized ? dispatch_bf16<true>(p, s) : dispatch_bf16<false>(p, s);
 }
 
 }  // namespace mhsa

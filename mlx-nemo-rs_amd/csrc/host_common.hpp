@@ -85,6 +85,7 @@ struct HostLinear {
 struct DevLinear {
   bool quantized = false;
   const void* w = nullptr;   // dense [N, K] (compute dtype) or u32 codes
+  const void* w16 = nullptr; // an fp32 copy's bf16 original, where w is one
   const float* sb = nullptr; // [N, K/64, 2]
   const float* bias = nullptr;
 };

@@ -22,6 +22,9 @@ struct GemmParams {
   const void* A = nullptr;
   int64_t lda = 0;
   const void* W = nullptr;
+  // fp32 activations of a bf16 module: the same weights in bf16 (W holds them
+  // widened to fp32), or null
+  const void* W16 = nullptr;
   const float* sb = nullptr;
   const float* bias = nullptr;
   const void* R = nullptr;

@@ -201,6 +201,7 @@ int32_t make_gemm(mhsa_layer* L, const DevLinear& lin, int n_rows_w, const void*
   p.A = A;
   p.lda = lda;
   p.W = lin.w;
+  p.W16 = lin.w16;
   p.sb = lin.sb;
   p.bias = lin.bias;
   p.R = R;
@@ -684,7 +685,10 @@ int32_t prepare_stream(mhsa_layer* L) {
       HIPCHK(L->wbuf32.ensure(host.size() * 4));
       HIPCHK(hipMemcpy(L->wbuf32.p, host.data(), host.size() * 4, hipMemcpyHostToDevice));
       for (int i = 0; i < 5; ++i)
-        if (!L->lin[i].quantized) L->sdev[i].w = static_cast<const float*>(L->wbuf32.p) + i * n;
+        if (!L->lin[i].quantized) {
+          L->sdev[i].w = static_cast<const float*>(L->wbuf32.p) + i * n;
+          L->sdev[i].w16 = L->dev[i].w;
+        }
     }
   }
   L->stream_version = L->version;
@@ -1120,6 +1124,7 @@ int32_t stream_step(mhsa_layer* L, mhsa_stream* S, const void* x, int B, int T, 
     fp.A = x;
     fp.lda = D;
     fp.W = L->sdev[0].w;
+    fp.W16 = L->sdev[0].w16;
     fp.sb = L->sdev[0].sb;
     fp.bias = L->sdev[0].bias;
     fp.C = q;

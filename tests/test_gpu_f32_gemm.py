@@ -1,0 +1,114 @@
+"""The fp32 projections on the bf16 matrix cores, where they can go wrong:
+remainders of their row tiles, one to many 64-column stages, every split of
+the contraction, each weight kind, and values that are not finite.
+
+The kernels write an fp32 value as the exact sum of three bf16 values and
+leave out products below 2^-22 of the whole one, so their results carry the
+error of fp32 sums: K 2^-24 |A| |W|^T per element at most (K roundings), and
+in the 2-norm that of K / 16 roundings of random sign.
+"""
+import numpy as np
+import pytest
+import torch
+
+import relpos_oracle as O
+import relpos_mhsa as M
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    M.library()
+    yield
+    torch.cuda.synchronize()
+
+
+def make_ff(rng, d, f, kind):
+    """(module, [W1, W2] in float64 as the kernels hold them)"""
+    w, dense = {}, []
+    for name, o, i in (("linear1", f, d), ("linear2", d, f)):
+        if kind == "u8":
+            codes = rng.integers(0, 256, size=(o, i))
+            sc = np.exp2(rng.uniform(-9, -7, size=(o, i // 64))).astype(np.float16)
+            bi = rng.uniform(-0.3, 0.1, size=(o, i // 64)).astype(np.float16)
+            w["f.%s.weight" % name], w["f.%s.scales" % name], w["f.%s.biases" % name] = W.pack_u8(codes), sc, bi
+            dense.append(O.dequantize(W.pack_u8(codes), sc, bi, 8, 64, O.F32).astype(np.float64))
+        else:
+            m = (rng.standard_normal((o, i)) / np.sqrt(i)).astype(np.float32)
+            w["f.%s.weight" % name] = m
+            dense.append((O.bf16_round(m) if kind == "bf16" else m).astype(np.float64))
+    m = M.FeedForward(d, f, False)
+    m.load_weights(w, "f")
+    m.set_dtype(O.BF16 if kind == "bf16" else O.F32)
+    return m, dense
+
+
+def check(got, x, w, what):
+    ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    k = x.shape[1]
+    err = np.abs(got.astype(np.float64) - ref)
+    assert (err <= k * 2.0 ** -24 * mag).all(), what
+    rel = np.linalg.norm(err) / np.linalg.norm(ref)
+    assert rel <= 2.0 ** -22 * max(1.0, np.sqrt(k / 1024)), f"{what}: {rel:.2e}"
+
+
+# 64-wide K is one stage; 513 and 1025 rows of 4096 columns are past the line
+# of the large tiles; the K-parallel kernel takes the few-row short-K ones
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("d,f,rows", [(64, 4096, 129), (128, 4096, 97), (192, 4096, 513), (192, 4096, 1025),
+                                      (1024, 1024, 351), (512, 4096, 577)])
+def test_linear1_tiles(d, f, rows, kind):
+    rng = np.random.default_rng(d + f + rows)
+    m, dense = make_ff(rng, d, f, kind)
+    x = rng.standard_normal((rows, d)).astype(np.float32)
+    got = m.debug_linear(0, torch.from_numpy(x).cuda()).cpu().numpy()
+    check(got, x.astype(np.float64), dense[0], f"linear1 {kind} {rows}x{f}x{d}")
+
+
+# K = 1088 .. 4096: one, two, four and eight splits, uneven ones among them
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("d,f,rows", [(64, 1088, 1), (128, 2048, 31), (64, 4096, 33), (1024, 4096, 14),
+                                      (1024, 4032, 225), (1024, 2048, 700), (1024, 4096, 1537)])
+def test_linear2_splits(d, f, rows, kind):
+    rng = np.random.default_rng(7 * d + f + rows)
+    m, dense = make_ff(rng, d, f, kind)
+    x = rng.standard_normal((rows, f)).astype(np.float32)
+    got = m.debug_linear(1, torch.from_numpy(x).cuda()).cpu().numpy()
+    check(got, x.astype(np.float64), dense[1], f"linear2 {kind} {rows}x{d}x{f}")
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("which,rows", [(0, 130), (1, 40)])
+def test_values_that_are_not_finite(which, rows, kind):
+    """Infinities, NaN and values that round to a bf16 infinity give what fp32
+    sums give, in their rows alone (one split and several)."""
+    rng = np.random.default_rng(rows)
+    m, dense = make_ff(rng, 128, 2048, kind)
+    k = 2048 if which else 128
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[3, 5], x[7, 9], x[11, 70], x[13, 1], x[13, 2] = np.inf, -np.inf, np.nan, np.inf, -np.inf
+    x[17, 100] = np.float32(3.4e38)
+    got = m.debug_linear(which, torch.from_numpy(x).cuda()).cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = x.astype(np.float64) @ dense[which].T
+        r32 = ref.astype(np.float32)
+    special = [3, 7, 11, 13, 17]
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(r32))
+    np.testing.assert_array_equal(np.where(np.isinf(r32), r32, 0), np.where(np.isinf(got), got, 0))
+    row = r32[17]
+    np.testing.assert_allclose(got[17][np.isfinite(row)], row[np.isfinite(row)], rtol=k * 2.0 ** -23)
+    rest = [r for r in range(rows) if r not in special]
+    check(got[rest], x[rest].astype(np.float64), dense[which], f"rows beside them, {kind}")
+
+
+@pytest.mark.parametrize("scale", [1e-20, 1e-3, 1e4, 1e18])
+def test_scaled_inputs(scale):
+    """The parts keep 24 bits over the fp32 range, not around 1 alone."""
+    rng = np.random.default_rng(5)
+    m, dense = make_ff(rng, 256, 4096, "f32")
+    x = (rng.standard_normal((160, 256)) * scale * np.exp2(rng.uniform(-12, 12, size=(160, 256)))).astype(np.float32)
+    got = m.debug_linear(0, torch.from_numpy(x).cuda()).cpu().numpy()
+    check(got, x.astype(np.float64), dense[0], f"scale {scale}")
