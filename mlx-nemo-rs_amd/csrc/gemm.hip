@@ -16,9 +16,9 @@
 //    one short utterance): persistent workgroups over 32 x 32 tiles, each
 //    tile's contraction split over the K / 64 waves of a workgroup and summed
 //    in LDS.
-//  * gemm_split_kernel + gemm_reduce: bf16 projections of few rows (the
-//    position table of a short utterance): K split over workgroups, the
-//    partial sums added in split order by a second kernel.
+//  * gemm_kw_kernel: bf16 projections of few output tiles (one utterance, a
+//    short position table), the contraction shared by the waves of a
+//    workgroup (gemm_kw_tile.hpp).
 //  * gemm_kernel: everything else (shapes and alignments the others do not
 //    take): BM x BN tiles on NWM x NWN waves, one 128-byte K step per LDS
 //    stage, double-buffered with a 16-byte row pad; an optional deterministic
@@ -42,6 +42,7 @@ constexpr int PITCH = ROWB + 16;  // LDS row pitch (bytes)
 
 #include "gemm_tile.hpp"
 #include "gemm_f32_tile.hpp"
+#include "gemm_kw_tile.hpp"
 
 template <typename T, bool QUANT, int BN, int NT>
 struct BLoad;
@@ -330,120 +331,6 @@ __global__ __launch_bounds__(256, 1) void gemm_pair_kernel(const GemmParams p1, 
 }
 
 // ---------------------------------------------------------------------------
-// Split-K kernel for projections with few rows (streaming chunks, short
-// utterances, the position table): too few output tiles to fill 256 CUs, so
-// the contraction is split. Workgroup (tile, z) takes a 64 x 64 output tile
-// over k-columns [z KS, (z + 1) KS), with KS the k-columns of one 512-byte LDS
-// row (128 fp32 or 256 bf16):
-//  * its whole A and B slices (64 rows x 512 bytes each) go to LDS in one
-//    burst of direct-to-LDS loads (quantized B: codes to registers,
-//    dequantised, written), so the workgroup waits on memory once;
-//  * 4 waves of 32 x 32 each, 16x16 MFMAs (fp32 16x16x4 or bf16 16x16x32),
-//    one 16-byte fragment per lane and operand per step; 16-byte chunk c of
-//    LDS row r sits at c ^ (r % 16), which spreads a fragment read's 16 rows
-//    over all 64 banks;
-//  * the raw fp32 sums go to partial[z][M][N], and gemm_reduce sums the
-//    splits in order z = 0, 1, ... and applies the epilogue. (Reducing in the
-//    last workgroup to arrive instead needs agent-scope fences, which on this
-//    chip write back and invalidate the whole L2 per workgroup: measured
-//    20x slower.)
-template <typename T, bool QUANT>
-__global__ __launch_bounds__(256) void gemm_split_kernel(const GemmParams p, int splits) {
-  constexpr int ES = sizeof(T);
-  constexpr int KS = 512 / ES;  // k-columns per workgroup
-  __shared__ __attribute__((aligned(1024))) char smem[2 * 64 * 512];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = w >> 1, wn = w & 1;
-  const int tile = (int)blockIdx.x / splits, z = (int)blockIdx.x % splits;
-  const int tilesN = p.N / 64;
-  const int m0 = tile / tilesN * 64, n0 = tile % tilesN * 64, k0 = z * KS;
-
-  // A rows [m0, M): 8 loads per wave of 64 x 16 bytes (rows past M read zero)
-  const char* Ab = reinterpret_cast<const char*>(p.A) + ((int64_t)m0 * p.lda + k0) * ES;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)Ab, (short)0, (int)(((int64_t)(p.M - m0) * p.lda - k0) * ES), kRawBuffer);
-#pragma unroll
-  for (int g = 0; g < 8; ++g) {
-    const int pos = (w * 8 + g) * 64 + lane, row = pos >> 5;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(smem + (w * 8 + g) * 1024), 16,
-                                             (int)(row * p.lda * ES + 16 * ((pos & 31) ^ (row & 15))), 0, 0, 0);
-  }
-  char* Bs = smem + 64 * 512;
-  if constexpr (!QUANT) {
-    const char* Bb = reinterpret_cast<const char*>(p.W) + ((int64_t)n0 * p.K + k0) * ES;
-    const __amdgpu_buffer_rsrc_t rb =
-        __builtin_amdgcn_make_buffer_rsrc((void*)Bb, (short)0, (int)(((int64_t)64 * p.K - k0) * ES), kRawBuffer);
-#pragma unroll
-    for (int g = 0; g < 8; ++g) {
-      const int pos = (w * 8 + g) * 64 + lane, row = pos >> 5;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void*)(Bs + (w * 8 + g) * 1024), 16,
-                                               (int)(row * p.K * ES + 16 * ((pos & 31) ^ (row & 15))), 0, 0, 0);
-    }
-  } else {
-    // 16 codes -> 16 values = ES 16-byte LDS chunks; KS / 16 code chunks per row
-    constexpr int CPR = KS / 16, QN = 64 * CPR / 256;
-    const unsigned char* Wq = reinterpret_cast<const unsigned char*>(p.W);
-    const int groups = p.K / 64;
-    u32x4 qr[QN];
-    floatx2 qs[QN];
-#pragma unroll
-    for (int i = 0; i < QN; ++i) {
-      const int q = tid + 256 * i, r = q / CPR, k = k0 + (q % CPR) * 16;
-      qr[i] = *reinterpret_cast<const u32x4*>(Wq + (int64_t)(n0 + r) * p.K + k);
-      qs[i] = *reinterpret_cast<const floatx2*>(p.sb + 2 * ((int64_t)(n0 + r) * groups + k / 64));
-    }
-#pragma unroll
-    for (int i = 0; i < QN; ++i) {
-      const int q = tid + 256 * i, r = q / CPR, cc = q % CPR;
-      T v[16];
-      dequant16<T>(qr[i], qs[i].x, qs[i].y, v);
-#pragma unroll
-      for (int e = 0; e < ES; ++e)
-        *reinterpret_cast<u32x4*>(Bs + r * 512 + 16 * ((cc * ES + e) ^ (r & 15))) = reinterpret_cast<const u32x4*>(v)[e];
-    }
-  }
-  __syncthreads();  // (waits for this wave's loads first)
-
-  // wave (wm, wn): rows 32 wm + 16 i + lane % 16 of A, 32 wn + 16 j + lane % 16
-  // of B; step s reads logical chunk 4 s + lane / 16 of each row
-  using F = typename Frag<T>::type;
-  floatx4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{};
-  const char* Ar = smem + (wm * 32 + (lane & 15)) * 512;
-  const char* Br = Bs + (wn * 32 + (lane & 15)) * 512;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const int off = 16 * ((4 * s + (lane >> 4)) ^ (lane & 15));
-    F a[2], b[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      a[t] = *reinterpret_cast<const F*>(Ar + t * 16 * 512 + off);
-      b[t] = *reinterpret_cast<const F*>(Br + t * 16 * 512 + off);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mma16(a[i], b[j], acc[i][j]);
-  }
-
-  // raw fp32 sums to partial[z][M][N]; gemm_reduce sums the splits in order
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + e;
-      if (row >= p.M) continue;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        p.partial[((int64_t)z * p.M + row) * p.N + n0 + wn * 32 + j * 16 + (lane & 15)] = acc[i][j][e];
-    }
-}
-
-// ---------------------------------------------------------------------------
 // fp32 projections with few rows (the streaming chunk's 224 rows, one short
 // utterance, the position table of a short one): too few 32 x 32 output
 // tiles to give every CU several, so each tile's contraction is split over
@@ -673,22 +560,6 @@ bool kpar_ok(const GemmParams& p) {
          (int64_t)((p.M + 31) / 32) * (p.N / 32) <= 4096;
 }
 
-// The split kernel applies when the scratch holds every split's sums and its
-// operand rows can be loaded as 16-byte chunks.
-template <typename T>
-int split_count(const GemmParams& p) {
-  constexpr int KS = 512 / (int)sizeof(T);
-  if (!p.partial || p.vt || p.K % KS || p.N % 64) return 0;
-  if ((p.lda * (int64_t)sizeof(T)) % 16 || (p.K * (int64_t)sizeof(T)) % 16) return 0;
-  if ((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W)) & 15) return 0;
-  if ((int64_t)p.M * p.lda * (int64_t)sizeof(T) >= ((int64_t)1 << 31) ||
-      (int64_t)p.N * p.K * (int64_t)sizeof(T) >= ((int64_t)1 << 31))
-    return 0;
-  const int splits = p.K / KS;
-  if ((int64_t)splits * p.M * p.N > p.partial_elems) return 0;
-  return splits;
-}
-
 // Estimated duration of one launch of the tile kernel, in units of one
 // 192 x 192 tile pass at K = 1024 with every CU busy (measured: a 256 x 256
 // pass 1.45; 128 x 128 0.5 alone on a CU with four stages, 0.75 for a pass of
@@ -727,10 +598,9 @@ bool tile_ok(const GemmParams& p) {
   return true;
 }
 
-// bf16 projections go to the tile kernel: with at least ~100 tiles of
-// 128 x 128 at the tile shape with the lowest estimated time, below that
-// (short inputs, a short position table) as 64 x 64 tiles with four stages
-// (749 x 1024 x 1024: 6.6 us against 12 us for split-K and its reduce).
+// bf16 projections past kw_form's line go to the tile kernel: with at least
+// ~100 tiles of 128 x 128 at the tile shape with the lowest estimated time,
+// below that as 64 x 64 tiles with four stages.
 // Stages: three (loads two ahead) for 192 x 192, 192 x 128 and the u8
 // 192 x 256; four for a 128 x 128 tile that has its CU to itself, two when
 // two share one; 256 x 256 and the dense 192 x 256 fit two. Returns false
@@ -738,7 +608,6 @@ bool tile_ok(const GemmParams& p) {
 bool tile_form(const GemmParams& p, TileForm& f) {
   if (!tile_ok(p) || p.N % 64) return false;
   if (p.N % 128 || m_tiles<128>(p) * (p.N / 128) < 96) {
-    if (m_tiles<64>(p) * (p.N / 64) < 16) return false;
     f = TileForm{64, 64, 4};
     return true;
   }
@@ -763,6 +632,47 @@ bool dispatch_tile(const GemmParams& p, hipStream_t s, hipError_t& err) {
   else if (f.ns == 4) err = launch_tile<128, 128, QUANT, 4>(p, s);
   else err = launch_tile<128, 128, QUANT, 2>(p, s);
   return true;
+}
+
+// Form of gemm_kw_kernel for one problem, or for two in one launch: 32 x 32
+// tiles, 64 x 32 or 64 x 64, the smallest that gives no CU a second tile (a
+// workgroup's LDS has the CU to itself, so a second round costs as much as
+// the first), 0 if none does. The forms sum in the same order. Measured, us a launch, 32 x 32 / 64 x 32 /
+// 64 x 64 against the 64 x 64 tile kernel:
+//   u8    125 x 1024 x 1024   4.4 /  5.0 /  6.8 against  8.6
+//         125 x 4096 x 1024   7.6 /  5.2 /  7.0 against  9.1
+//         203 x 4096 x 1024  13.0 /  8.9 /  7.2 against  9.7
+//         203 x 1024 x 4096   9.1 / 10.2 / 15.2 against 24.3
+//         700 x 1024 x 4096  24.2 / 22.3 / 17.8 against 25.5
+//   bf16  125 x 1024 x 1024   4.1 /  4.9 /  6.4 against  5.8
+//         400 x 1024 x 4096  14.5 / 10.6 / 14.4 against 15.0
+//         203 x 4096 x 1024  12.5 /  8.9 /  7.2 against  6.7
+// so one dense problem does not take the 64 x 64 form (the tile kernel's
+// four waves are as fast where nothing is dequantised), but a pair does: it
+// saves a launch of 4 us.
+template <bool QUANT>
+int kw_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
+  if (p1.one_chain || !tile_ok(p1) || p1.N % 64) return 0;
+  const int64_t cus = device_cus();
+  auto tiles = [&](auto count) { return count(p1) + (p2 ? count(*p2) : 0); };
+  if (tiles([](const GemmParams& p) { return m_tiles<32>(p) * (p.N / 32); }) <= cus) return 1;
+  if (tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 32); }) <= cus) return 2;
+  if ((QUANT || p2) && tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 64); }) <= cus) return 3;
+  return 0;
+}
+
+template <bool QUANT>
+hipError_t launch_kw(int form, const GemmParams& p1, const GemmParams* p2, hipStream_t s) {
+  auto go = [&](auto kernel, int64_t t1, int64_t t2) {
+    const int n1 = (int)((t1 + 7) / 8 * 8), n2 = (int)((t2 + 7) / 8 * 8);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(n1 + n2)), dim3(512), 0, s, p1, n1, p2 ? *p2 : p1);
+    return hipGetLastError();
+  };
+  if (form == 1)
+    return go(gemm_kw_kernel<1, 1, 8, 2, QUANT>, m_tiles<32>(p1) * (p1.N / 32), p2 ? m_tiles<32>(*p2) * (p2->N / 32) : 0);
+  if (form == 2)
+    return go(gemm_kw_kernel<2, 1, 8, 1, QUANT>, m_tiles<64>(p1) * (p1.N / 32), p2 ? m_tiles<64>(*p2) * (p2->N / 32) : 0);
+  return go(gemm_kw_kernel<2, 2, 8, 1, QUANT>, m_tiles<64>(p1) * (p1.N / 64), p2 ? m_tiles<64>(*p2) * (p2->N / 64) : 0);
 }
 
 template <typename T, bool QUANT, int BM, int BN, int NWM, int NWN>
@@ -854,6 +764,7 @@ template <bool QUANT>
 hipError_t dispatch_bf16(const GemmParams& p, hipStream_t s) {
   using T = bf16;
   hipError_t err;
+  if (const int form = kw_form<QUANT>(p)) return launch_kw<QUANT>(form, p, nullptr, s);
   if (dispatch_tile<QUANT>(p, s, err)) return err;
   // 256x256 (8 waves) when it still fills the GPU about twice over: it
   // halves the LDS and L2 traffic per flop of 128x128 (measured 1.15x on
@@ -863,18 +774,6 @@ hipError_t dispatch_bf16(const GemmParams& p, hipStream_t s) {
     return launch<T, QUANT, 256, 256, 4, 2>(p, 1, s);
   if (m_tiles<128>(p) * (p.N / 128) >= 384 && p.N % 128 == 0) return launch<T, QUANT, 128, 128, 2, 2>(p, 1, s);
   if (p.vt) return launch<T, QUANT, 128, 128, 2, 2>(p, 1, s);  // V^T epilogue needs whole 128-row tiles
-  // few rows (the position table of a short utterance)
-  if (const int splits = split_count<T>(p)) {
-    const int64_t tiles = (int64_t)((p.M + 63) / 64) * (p.N / 64);
-    hipLaunchKernelGGL((gemm_split_kernel<T, QUANT>), dim3((unsigned)(tiles * splits)), dim3(256), 0, s, p, splits);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // (also for one split: the reduce kernel applies the epilogue)
-    const int64_t total = (int64_t)p.M * p.N;
-    const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 4096);
-    hipLaunchKernelGGL(gemm_reduce<T>, dim3(blocks), dim3(256), 0, s, p, splits);
-    return hipGetLastError();
-  }
   return launch<T, QUANT, 64, 64, 2, 2>(p, small_splits<T>(p), s);
 }
 
@@ -905,7 +804,8 @@ hipError_t gemm_check(DType dt, bool quantized, const GemmParams& p) {
 }
 
 bool gemm_tile_form(DType dt, bool quantized, const GemmParams& p, TileForm& f) {
-  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess && tile_form(p, f);
+  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess &&
+         !gemm_few_tiles(dt, quantized, p) && tile_form(p, f);
 }
 
 namespace {
@@ -941,14 +841,28 @@ int device_cus() {
   return n;
 }
 
+bool gemm_few_tiles(DType dt, bool quantized, const GemmParams& p) {
+  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess &&
+         (quantized ? kw_form<true>(p) : kw_form<false>(p));
+}
+
 // Paired where p1's tiles take one round of CUs: the CUs its slowest tiles
 // leave idle then run p2's tiles (measured: 3000 x 3072 Q/K/V tiles with
 // 749 x 1024 position tiles, step 0.064 -> 0.061 ms). Past one round it
 // measured no gain (15000 x 3072 with 257 rows: step 0.2174 against
-// 0.2202 ms).
+// 0.2202 ms). Two problems of few tiles share a launch of gemm_kw_kernel
+// where one round holds both.
+namespace {
+int pair_kw_form(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
+  if (!gemm_few_tiles(dt, quantized, p1) || !gemm_few_tiles(dt, quantized, p2)) return 0;
+  return quantized ? kw_form<true>(p1, &p2) : kw_form<false>(p1, &p2);
+}
+}  // namespace
+
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
+  if (pair_kw_form(dt, quantized, p1, p2)) return true;
   TileForm f1, f2;
-  return p1.M > 0 && p2.M > 0 && gemm_tile_form(dt, quantized, p1, f1) && f1.bm != 64 &&
+  return gemm_tile_form(dt, quantized, p1, f1) && f1.bm != 64 &&
          gemm_tile_form(dt, quantized, p2, f2) && f2.bm == 64 &&
          (p1.seg_T > 0 ? (int64_t)(p1.M / p1.seg_T) * ((p1.seg_T + f1.bm - 1) / f1.bm) : (p1.M + f1.bm - 1) / f1.bm) *
                  (p1.N / f1.bn) <=
@@ -957,6 +871,8 @@ bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmPara
 
 hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2, hipStream_t s) {
   if (!gemm_pair_ok(dt, quantized, p1, p2)) return hipErrorInvalidValue;
+  if (const int form = pair_kw_form(dt, quantized, p1, p2))
+    return quantized ? launch_kw<true>(form, p1, &p2, s) : launch_kw<false>(form, p1, &p2, s);
   TileForm f;
   tile_form(p1, f);
   return quantized ? dispatch_pair<true>(f, p1, p2, s) : dispatch_pair<false>(f, p1, p2, s);
