@@ -157,8 +157,9 @@ int32_t ffn_impl(mhsa_ffn* f, const void* x, int rows, void* out, const void* re
   return MHSA_OK;
 }
 
-int32_t ffn_sublayer(mhsa_ffn* f, void* x, int32_t rows, const float* gamma, const float* beta, float eps, DType act,
-                     hipStream_t s) {
+// x <- x0 + 0.5 FF(LayerNorm(x0)); x0 is x or does not overlap it.
+int32_t ffn_sublayer(mhsa_ffn* f, const void* x0, void* x, int32_t rows, const float* gamma, const float* beta,
+                     float eps, DType act, hipStream_t s) {
   if (!x || rows <= 0) return fail(MHSA_EINVAL, "bad sublayer arguments");
   if (!aligned16(x)) return fail(MHSA_EINVAL, "device tensors must be 16-byte aligned");
   if (f->D > mhsa::kMaxLayerNormDim)
@@ -187,7 +188,7 @@ int32_t ffn_sublayer(mhsa_ffn* f, void* x, int32_t rows, const float* gamma, con
   {
     ProfScope ps(f->prof, "layer_norm", s);
     for (int r = ps.reps(); r > 0; --r)
-      HIPCHK(mhsa::layer_norm(act, x, f->hbuf.p, gd, bd, eps, rows, D, s));
+      HIPCHK(mhsa::layer_norm(act, x0, f->hbuf.p, gd, bd, eps, rows, D, s, 0, x0 != x ? x : nullptr, act));
   }
   // x + 0.5 * FF(LN(x)): the half step scales exactly (conformer.rs:1727-1729)
   return ffn_impl(f, f->hbuf.p, rows, x, x, 0.5f, act, s);
@@ -259,13 +260,13 @@ int32_t mhsa_ffn_forward_f32(mhsa_ffn* f, const float* x, int32_t rows, float* o
 int32_t mhsa_ffn_sublayer_forward(mhsa_ffn* f, void* x, int32_t rows, const float* gamma, const float* beta, float eps,
                                   void* hs) {
   if (!f) return fail(MHSA_EINVAL, "null handle");
-  return ffn_sublayer(f, x, rows, gamma, beta, eps, f->dt, static_cast<hipStream_t>(hs));
+  return ffn_sublayer(f, x, x, rows, gamma, beta, eps, f->dt, static_cast<hipStream_t>(hs));
 }
 
 int32_t mhsa_ffn_sublayer_forward_f32(mhsa_ffn* f, float* x, int32_t rows, const float* gamma, const float* beta,
                                       float eps, void* hs) {
   if (!f) return fail(MHSA_EINVAL, "null handle");
-  return ffn_sublayer(f, x, rows, gamma, beta, eps, mhsa::kF32, static_cast<hipStream_t>(hs));
+  return ffn_sublayer(f, x, x, rows, gamma, beta, eps, mhsa::kF32, static_cast<hipStream_t>(hs));
 }
 
 int32_t mhsa_ffn_profile_enable(mhsa_ffn* f, int32_t enable) {
@@ -573,6 +574,12 @@ int32_t conv_sublayer_norm(mhsa_conv* m, const float* gamma, const float* beta, 
 
 }  // namespace
 
+int32_t mhsa_ffn_sublayer_from(mhsa_ffn* f, const void* x0, void* x, int rows, const float* gamma, const float* beta,
+                               float eps, DType act, hipStream_t s) {
+  if (!x0 || !aligned16(x0)) return fail(MHSA_EINVAL, "device tensors must be 16-byte aligned and not null");
+  return ffn_sublayer(f, x0, x, rows, gamma, beta, eps, act, s);
+}
+
 int32_t mhsa_conv_sublayer_to_f32(mhsa_conv* m, const void* x, DType x_dt, int B, int T, const int32_t* lens,
                                   const float* gamma, const float* beta, float eps, float* out, hipStream_t s) {
   if (int32_t rc = check_conv(m)) return rc;
@@ -591,9 +598,7 @@ int32_t mhsa_conv_sublayer_to_f32(mhsa_conv* m, const void* x, DType x_dt, int B
   HIPCHK(m->hbuf.ensure(align_up(rows * D * mhsa::dtype_size(x_dt), 256)));
   // conv_norm in the activations' dtype (conformer.rs:1793); the residual x
   // (conformer.rs:1814) then goes to out in f32, where the module adds to it
-  HIPCHK(mhsa::layer_norm(x_dt, x, m->hbuf.p, gd, bd, eps, (int)rows, D, s));
-  if (x_dt != mhsa::kF32) HIPCHK(mhsa::widen_bf16(x, out, rows * D, s));
-  else if (x != out) HIPCHK(hipMemcpyAsync(out, x, (size_t)rows * D * 4, hipMemcpyDeviceToDevice, s));
+  HIPCHK(mhsa::layer_norm(x_dt, x, m->hbuf.p, gd, bd, eps, (int)rows, D, s, 0, x != out ? out : nullptr, mhsa::kF32));
   return conv_impl(m, m->hbuf.p, B, T, x_dt, lens, nullptr, out, out, s);
 }
 

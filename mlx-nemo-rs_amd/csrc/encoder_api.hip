@@ -94,7 +94,8 @@ int32_t load_norm(const TensorMap& m, const std::string& prefix, int D, std::vec
   return MHSA_OK;
 }
 
-int32_t block_forward(mhsa_block* k, void* x, int B, int T, const void* pos_emb, int pos_len,
+// x <- the block of x0 (x itself or not overlapping it).
+int32_t block_forward(mhsa_block* k, const void* x0, void* x, int B, int T, const void* pos_emb, int pos_len,
                       const mhsa_context* ctx, const int32_t* lens, hipStream_t s) {
   if (!x || !pos_emb || B <= 0 || T <= 0) return fail(MHSA_EINVAL, "bad block arguments");
   if (k->causal && k->dt == mhsa::kBF16)
@@ -102,7 +103,7 @@ int32_t block_forward(mhsa_block* k, void* x, int B, int T, const void* pos_emb,
                               "input cannot hold in place: call mhsa_block_forward_to");
   const int rows = B * T;
   // conformer.rs:1703-1729, 1747-1780, 1790-1814, 1827-1851, 1862
-  if (int32_t rc = mhsa_ffn_sublayer_forward(k->ff1, x, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, s))
+  if (int32_t rc = mhsa_ffn_sublayer_from(k->ff1, x0, x, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, k->dt, s))
     return rc;
   if (int32_t rc = mhsa_sublayer_forward(k->attn, x, B, T, k->nw[1].data(), k->nb[1].data(), kNormEps, pos_emb,
                                          pos_len, ctx, lens, s))
@@ -127,13 +128,14 @@ DType block_out_dtype(const mhsa_block* k, DType xdt) {
 }
 
 // The block on activations made f32 before it (a bf16 block's ops then all
-// run in f32 on the parameters' bf16 values), in place on x:
+// run in f32 on the parameters' bf16 values), from x0 to x as block_forward:
 // conformer.rs:1703-1729, 1747-1780, 1790-1814, 1827-1851, 1862 as MLX
 // promotes them.
-int32_t block_forward_act32(mhsa_block* k, float* x, int B, int T, const void* pos_emb, int pos_len,
+int32_t block_forward_act32(mhsa_block* k, const float* x0, float* x, int B, int T, const void* pos_emb, int pos_len,
                             const mhsa_context* ctx, const int32_t* lens, hipStream_t s) {
   const int rows = B * T;
-  if (int32_t rc = mhsa_ffn_sublayer_forward_f32(k->ff1, x, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, s))
+  if (int32_t rc = mhsa_ffn_sublayer_from(k->ff1, x0, x, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, mhsa::kF32,
+                                          s))
     return rc;
   if (int32_t rc = mhsa_sublayer_forward_act32(k->attn, x, B, T, k->nw[1].data(), k->nb[1].data(), kNormEps,
                                                pos_emb, pos_len, ctx, lens, s))
@@ -167,18 +169,16 @@ int32_t block_forward_to(mhsa_block* k, const void* x, DType xdt, int B, int T, 
   if (out != x && xb < ob + out_bytes && ob < xb + in_bytes)
     return fail(MHSA_EINVAL, "x and out must be the same buffer or not overlap");
   if (odt == xdt) {
-    if (out != x) HIPCHK(hipMemcpyAsync(out, x, in_bytes, hipMemcpyDeviceToDevice, s));
-    if (xdt == k->dt) return block_forward(k, out, B, T, pos_emb, pos_len, ctx, lens, s);
-    return block_forward_act32(k, static_cast<float*>(out), B, T, pos_emb, pos_len, ctx, lens, s);
+    if (xdt == k->dt) return block_forward(k, x, out, B, T, pos_emb, pos_len, ctx, lens, s);
+    return block_forward_act32(k, static_cast<const float*>(x), static_cast<float*>(out), B, T, pos_emb, pos_len, ctx,
+                               lens, s);
   }
   // bf16 activations into a causal bf16 block: bf16 up to the conv's padding
   if (out == x) return fail(MHSA_EINVAL, "the f32 output cannot overwrite its bf16 input (x and out must not overlap)");
-  if (x != k->work.p) {  // (the encoder loop may have put them there)
-    HIPCHK(k->work.ensure(align_up((int64_t)in_bytes, 256)));
-    HIPCHK(hipMemcpyAsync(k->work.p, x, in_bytes, hipMemcpyDeviceToDevice, s));
-  }
+  if (x != k->work.p) HIPCHK(k->work.ensure(align_up((int64_t)in_bytes, 256)));  // (the encoder loop may have put x there)
   const int rows = B * T;
-  if (int32_t rc = mhsa_ffn_sublayer_forward(k->ff1, k->work.p, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, s))
+  if (int32_t rc = mhsa_ffn_sublayer_from(k->ff1, x, k->work.p, rows, k->nw[0].data(), k->nb[0].data(), kNormEps, k->dt,
+                                          s))
     return rc;
   if (int32_t rc = mhsa_sublayer_forward(k->attn, k->work.p, B, T, k->nw[1].data(), k->nb[1].data(), kNormEps,
                                          pos_emb, pos_len, ctx, lens, s))
@@ -289,7 +289,7 @@ mhsa_conv* mhsa_block_conv(mhsa_block* k) { return k ? k->conv : nullptr; }
 int32_t mhsa_block_forward(mhsa_block* k, void* x, int32_t batch, int32_t seq_len, const void* pos_emb,
                            int32_t pos_len, const mhsa_context* ctx, const int32_t* lengths, void* hs) {
   if (int32_t rc = check_block(k)) return rc;
-  return block_forward(k, x, batch, seq_len, pos_emb, pos_len, ctx, lengths, static_cast<hipStream_t>(hs));
+  return block_forward(k, x, x, batch, seq_len, pos_emb, pos_len, ctx, lengths, static_cast<hipStream_t>(hs));
 }
 
 int32_t mhsa_encoder_forward(mhsa_block* const* blocks, int32_t n_layers, void* x, int32_t batch, int32_t seq_len,
@@ -303,7 +303,7 @@ int32_t mhsa_encoder_forward(mhsa_block* const* blocks, int32_t n_layers, void* 
   }
   // one pos_emb, context and padding for every layer (conformer.rs:542-550)
   for (int l = 0; l < n_layers; ++l)
-    if (int32_t rc = block_forward(blocks[l], x, batch, seq_len, pos_emb, pos_len, ctx, lengths,
+    if (int32_t rc = block_forward(blocks[l], x, x, batch, seq_len, pos_emb, pos_len, ctx, lengths,
                                    static_cast<hipStream_t>(hs)))
       return rc;
   return MHSA_OK;

@@ -180,10 +180,12 @@ hipError_t export_pos_index(int T, int L, int qoff, int center, int32_t* out, hi
 // y = T(LayerNorm(x) * gamma + beta), statistics in fp32; gamma/beta may be null.
 // act = kActSilu then applies nn::silu to the stored result (the conv
 // module's norm -> SiLU). Rows are held in registers, one wave per row:
-// D <= kMaxLayerNormDim; y may alias x.
+// D <= kMaxLayerNormDim; y may alias x. With `copy` (neither x nor y), x also
+// goes there in copy_dt: dt, or f32.
 constexpr int kMaxLayerNormDim = 2048;
 hipError_t layer_norm(DType dt, const void* x, void* y, const float* gamma, const float* beta,
-                      float eps, int rows, int D, hipStream_t s, int act = 0);
+                      float eps, int rows, int D, hipStream_t s, int act = 0, void* copy = nullptr,
+                      DType copy_dt = kF32);
 
 // ConvolutionModule middle (conformer.rs:2197-2291, 2305-2378) for a batch
 // chunk: y[b, t, c] = post(sum_k w[k, c] * u[b, t - left + k, c] (+ bias[c]))

@@ -13,10 +13,14 @@
 namespace mhsa {
 namespace {
 
-// One wave per row; two-pass statistics in fp32 from registers.
+// One wave per row; two-pass statistics in fp32 from registers. With `copy`,
+// the row as it came also goes there, in T or widened to f32: a sublayer that
+// does not run in place needs its input as the residual, and the row is at
+// hand (a copy or widening pass of its own took 5 us at 3000 x 1024 bf16; the
+// extra store costs the LayerNorm under 1).
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void ln_kernel(const T* x, T* y, const float* gamma, const float* beta,
-                                                 float eps, int rows, int D, int act) {
+                                                 float eps, int rows, int D, int act, void* copy, bool copy32) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -28,6 +32,10 @@ __global__ __launch_bounds__(256) void ln_kernel(const T* x, T* y, const float* 
     const int c = lane + 64 * i;
     v[i] = c < D ? (float)xr[c] : 0.f;
     s += v[i];
+    if (copy && c < D) {
+      if (copy32) reinterpret_cast<float*>(copy)[(int64_t)row * D + c] = v[i];
+      else reinterpret_cast<T*>(copy)[(int64_t)row * D + c] = from_float<T>(v[i]);
+    }
   }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   const float mean = s / (float)D;
@@ -58,7 +66,7 @@ __global__ __launch_bounds__(256) void ln_kernel(const T* x, T* y, const float* 
 // (D a multiple of 64 chunks), gamma and beta read as float4.
 template <typename T, int NCH, bool GAMMA, bool BETA>
 __global__ __launch_bounds__(256) void ln_vec_kernel(const T* x, T* y, const float* gamma, const float* beta,
-                                                     float eps, int rows, int D, int act) {
+                                                     float eps, int rows, int D, int act, void* copy, bool copy32) {
   constexpr int E = 16 / sizeof(T);  // elements per chunk
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -90,6 +98,20 @@ __global__ __launch_bounds__(256) void ln_vec_kernel(const T* x, T* y, const flo
     for (int e = 0; e < E; ++e) {
       v[j][e] = (float)t[e];
       s += v[j][e];
+    }
+  }
+  if (copy) {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const int64_t at = (int64_t)row * D + (lane + 64 * j) * E;
+      if (copy32) {
+#pragma unroll
+        for (int e = 0; e < E; e += 4)
+          *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(copy) + at + e) =
+              floatx4{v[j][e], v[j][e + 1], v[j][e + 2], v[j][e + 3]};
+      } else {
+        *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(copy) + at) = raw[j];
+      }
     }
   }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -132,39 +154,47 @@ __global__ __launch_bounds__(256) void ln_vec_kernel(const T* x, T* y, const flo
 
 template <typename T, int NCH>
 hipError_t ln_vec_launch(dim3 grid, const T* x, T* y, const float* g, const float* b, float eps, int rows, int D,
-                         int act, hipStream_t s) {
-  if (g && b) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, true, true>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act);
-  else if (g) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, true, false>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act);
-  else if (b) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, false, true>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act);
-  else hipLaunchKernelGGL((ln_vec_kernel<T, NCH, false, false>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act);
+                         int act, void* copy, bool copy32, hipStream_t s) {
+  if (g && b) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, true, true>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act, copy,
+                                 copy32);
+  else if (g) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, true, false>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act, copy,
+                                 copy32);
+  else if (b) hipLaunchKernelGGL((ln_vec_kernel<T, NCH, false, true>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act, copy,
+                                 copy32);
+  else hipLaunchKernelGGL((ln_vec_kernel<T, NCH, false, false>), grid, dim3(256), 0, s, x, y, g, b, eps, rows, D, act, copy,
+                                 copy32);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t ln_launch(const void* x, void* y, const float* g, const float* b, float eps, int rows, int D, int act,
-                     hipStream_t s) {
+                     void* copy, bool copy32, hipStream_t s) {
   dim3 grid((rows + 3) / 4);
   constexpr int E = 16 / sizeof(T);
   const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
-                         reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+                         reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(b) |
+                         reinterpret_cast<uintptr_t>(copy)) & 15) == 0;
   if (aligned && D % (64 * E) == 0) {
     switch (D / (64 * E)) {
       case 1:
-        return ln_vec_launch<T, 1>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, s);
+        return ln_vec_launch<T, 1>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, copy, copy32, s);
       case 2:
-        return ln_vec_launch<T, 2>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, s);
+        return ln_vec_launch<T, 2>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, copy, copy32, s);
       case 4:
-        return ln_vec_launch<T, 4>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, s);
+        return ln_vec_launch<T, 4>(grid, (const T*)x, (T*)y, g, b, eps, rows, D, act, copy, copy32, s);
       default:
         break;
     }
   }
   if (D <= 512)
-    hipLaunchKernelGGL((ln_kernel<T, 8>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act);
+    hipLaunchKernelGGL((ln_kernel<T, 8>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act,
+                       copy, copy32);
   else if (D <= 1024)
-    hipLaunchKernelGGL((ln_kernel<T, 16>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act);
+    hipLaunchKernelGGL((ln_kernel<T, 16>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act,
+                       copy, copy32);
   else
-    hipLaunchKernelGGL((ln_kernel<T, 32>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act);
+    hipLaunchKernelGGL((ln_kernel<T, 32>), grid, dim3(256), 0, s, (const T*)x, (T*)y, g, b, eps, rows, D, act,
+                       copy, copy32);
   return hipGetLastError();
 }
 
@@ -240,11 +270,13 @@ hipError_t fill_zero(void* ptr, size_t bytes, hipStream_t s) {
 }
 
 hipError_t layer_norm(DType dt, const void* x, void* y, const float* gamma, const float* beta, float eps, int rows,
-                      int D, hipStream_t s, int act) {
+                      int D, hipStream_t s, int act, void* copy, DType copy_dt) {
   if (rows <= 0) return hipSuccess;
   if (!x || !y || D <= 0 || D > kMaxLayerNormDim) return hipErrorInvalidValue;
-  return dt == kF32 ? ln_launch<float>(x, y, gamma, beta, eps, rows, D, act, s)
-                    : ln_launch<bf16>(x, y, gamma, beta, eps, rows, D, act, s);
+  if (copy && (copy == y || (copy_dt != kF32 && copy_dt != dt))) return hipErrorInvalidValue;
+  const bool c32 = copy_dt == kF32;
+  return dt == kF32 ? ln_launch<float>(x, y, gamma, beta, eps, rows, D, act, copy, c32, s)
+                    : ln_launch<bf16>(x, y, gamma, beta, eps, rows, D, act, copy, c32, s);
 }
 
 static hipError_t ring_copy(DType dt, const void* src, void* dst, int B, int n, int D, int R, int64_t ld, int off,

@@ -20,6 +20,12 @@ int32_t mhsa_sublayer_forward_act32(mhsa_layer* L, float* x, int B, int T, const
                                     float eps, const void* pos_emb, int pos_len, const mhsa_context* ctx,
                                     const int32_t* lens, hipStream_t s);
 
+// x <- x0 + 0.5 FF(LayerNorm(x0)) (conformer.rs:1703-1729) on activations of
+// dtype `act`, the module's or f32: the first sublayer of a block that does
+// not run in place. x0 is x or does not overlap it. (block_api.hip)
+int32_t mhsa_ffn_sublayer_from(mhsa_ffn* f, const void* x0, void* x, int rows, const float* gamma, const float* beta,
+                               float eps, mhsa::DType act, hipStream_t s);
+
 // out = x + conv(LayerNorm(x)) offline in f32 (conformer.rs:1790-1814): x
 // [B, T, D] in x_dt, either f32 activations or, for a causal module, bf16
 // ones in a bf16 module, whose LayerNorm, pointwise_conv1 and GLU stay bf16
