@@ -99,6 +99,8 @@ __host__ __device__ inline void key_range(const AttnParams& p, int bl, int i0, i
   }
 }
 
+#include "attention_f32_tile.hpp"
+
 template <typename T, int DK, int NW, int NKO = 0>
 struct Cfg {
   static constexpr int NT = 64 * NW;
@@ -1437,6 +1439,11 @@ hipError_t dispatch_nw(const AttnParams& p, int nb, hipStream_t s) {
   if constexpr (sizeof(T) == 4) {
     if (!dbg && (p.T <= 16 || (int64_t)nb * p.H * ((p.T + 63) / 64) < 128))
       return launch_ks<T, DK, 4>(p, nb, s);  // (per-wave tiles: 34 / 37 KB of LDS)
+    if (!dbg) {
+      hipLaunchKernelGGL((attn_f32_kernel<DK>), dim3(p.H, (p.T + 63) / 64, nb), dim3(256), 0, s, p);
+      count_form(kFormGeneric);
+      return hipGetLastError();
+    }
   }
   return dbg ? launch<T, DK, 4, true>(p, nb, s) : launch<T, DK, 4, false>(p, nb, s);
 }

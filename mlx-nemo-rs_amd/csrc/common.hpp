@@ -93,6 +93,32 @@ __device__ __forceinline__ float silu_value(float v) {
   return round_to<T>(v * sigmoid_value<T>(v));
 }
 
+// An fp32 value is the exact sum of three bf16 values, x = h + m + l: h is x
+// cut to its top 8 significant bits, m the remainder (under 2^-7 |x|) rounded
+// to bf16, and what is left, l, under 2^-15 |x|, fits bf16. This splits a
+// pair, packed as MFMA operands take them. (Parts below the smallest bf16
+// subnormal are lost: values under ~1e-33 keep fewer bits. An infinite or NaN
+// value makes m and l NaN, and so every sum it enters: the kernels recompute
+// those in plain fp32.)
+// (The empty asm keeps the packed word opaque: otherwise the compiler
+// converts each value once more for the subtractions.)
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  const bf16x2 v = {(bf16)a, (bf16)b};
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  asm("" : "+v"(u));
+  return u;
+}
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+  a -= __builtin_bit_cast(float, ua & 0xFFFF0000u);
+  b -= __builtin_bit_cast(float, ub & 0xFFFF0000u);
+  m = pack_bf16(a, b);
+  a -= __builtin_bit_cast(float, m << 16);
+  b -= __builtin_bit_cast(float, m & 0xFFFF0000u);
+  l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+
 template <typename T> __device__ __forceinline__ typename Frag<T>::type zero_frag();
 template <> __device__ __forceinline__ floatx4 zero_frag<float>() { return floatx4{0.f, 0.f, 0.f, 0.f}; }
 template <> __device__ __forceinline__ bf16x8 zero_frag<bf16>() {

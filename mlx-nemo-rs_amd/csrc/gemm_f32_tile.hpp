@@ -3,31 +3,6 @@
 // common.hpp, kernels.hpp, quant.hpp and gemm_tile.hpp.
 #pragma once
 
-// An fp32 value is the exact sum of three bf16 values, x = h + m + l (8
-// significant bits each, every part rounded to nearest, so |m| <= 2^-8 |x|
-// and |l| <= 2^-16 |x|). This splits 8 of them, packed as MFMA fragments.
-// (Parts below the smallest bf16 subnormal are lost: values under ~1e-33
-// keep fewer bits. An infinite or NaN value, or one that rounds to a bf16
-// infinity, makes every sum it enters NaN; the epilogue recomputes those.)
-// (The empty asm keeps the packed word opaque: otherwise the compiler
-// converts each value once more for the subtractions.)
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  const bf16x2 v = {(bf16)a, (bf16)b};
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  asm("" : "+v"(u));
-  return u;
-}
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-  h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-  a -= __builtin_bit_cast(float, ua & 0xFFFF0000u);
-  b -= __builtin_bit_cast(float, ub & 0xFFFF0000u);
-  m = pack_bf16(a, b);
-  a -= __builtin_bit_cast(float, m << 16);
-  b -= __builtin_bit_cast(float, m & 0xFFFF0000u);
-  l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
-}
-
 enum WKind { kWF32 = 0, kWBF16 = 1, kWU8 = 2 };
 
 // A[row, :] . W[col, :] in plain fp32 (the epilogue's recomputation).

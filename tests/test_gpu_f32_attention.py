@@ -1,0 +1,78 @@
+"""The offline fp32 attention on the bf16 matrix cores, where it can go wrong:
+query blocks and key tiles that end inside a tile, one tile to many turns of
+the position ring, contexts that start inside a block, items of different
+lengths, and values that are not finite.
+
+The products left out are below 2^-22 of the whole one, and the sums are fp32:
+the error in the 2-norm is that of the projections and the attention at a few
+roundings of random sign each, 2^-19 at most (measured 2^-21).
+"""
+import numpy as np
+import pytest
+import torch
+
+import relpos_oracle as O
+import relpos_mhsa as M
+import workloads as W
+from _util import oracle_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    M.library()
+    yield
+    torch.cuda.synchronize()
+
+
+def make(d, h, T, seed):
+    rng = np.random.default_rng(seed)
+    w = W.make_layer_weights(rng, d, h, True, False)
+    layer = M.RelPositionMultiHeadAttention(d, h, True)
+    layer.load_weights(W.prefixed(w, "l"), "l")
+    layer.set_dtype(O.F32)
+    return rng, layer, oracle_params(w, d, h), O.RelPositionalEncoding(d, 5000, True).get_encoding(T)
+
+
+def forward(layer, x, pos, ctx, lengths, T):
+    before = M.debug_attention_forms()
+    got = layer.forward(torch.from_numpy(x).cuda(), torch.from_numpy(pos).float().cuda().contiguous(), ctx,
+                        M.key_padding_mask(lengths, T)).cpu().numpy().astype(np.float64)
+    after = M.debug_attention_forms()
+    assert {k for k in after if after[k] > before[k]} == {"generic"}
+    return got
+
+
+@pytest.mark.parametrize("d,h,B,T,ctx", [
+    (512, 8, 16, 17, None), (512, 8, 16, 64, None), (256, 2, 64, 33, None), (256, 2, 32, 65, ((5, 40), "regular")),
+    (512, 8, 4, 225, ((30, 0), "regular")), (1024, 8, 3, 353, None), (1024, 8, 3, 353, ((70, 13), "chunked_limited")),
+    (256, 2, 16, 200, ((100, -1), "regular"))])
+def test_forward_against_oracle(d, h, B, T, ctx):
+    rng, layer, p, pos = make(d, h, T, d + B + T)
+    x = rng.standard_normal((B, T, d)).astype(np.float32)
+    lengths = [T] + [max(1, T - 1 - 37 * i % T) for i in range(1, B)]
+    got = forward(layer, x, pos, M.AttentionContext.new(*ctx) if ctx else None, lengths, T)
+    for b in sorted({0, 1, B - 1}):
+        ref = O.mhsa_forward(p, x[b:b + 1], pos, O.AttentionContext.new(*ctx) if ctx else None,
+                             O.key_padding_mask([lengths[b]], T), O.F32)
+        rows = np.isfinite(ref).all(axis=-1)
+        err = np.linalg.norm(got[b:b + 1][rows] - ref[rows]) / np.linalg.norm(ref[rows])
+        assert rows.any() and err < 2.0 ** -19, (b, err)
+
+
+def test_values_that_are_not_finite():
+    """A frame of infinities behind an item's end hides from its queries, and
+    the other items do not see it."""
+    d, h, B, T = 512, 8, 16, 100
+    rng, layer, p, pos = make(d, h, T, 5)
+    x = rng.standard_normal((B, T, d)).astype(np.float32)
+    lengths = [70] * B
+    clean = forward(layer, x, pos, None, lengths, T)
+    x[3, 75] = np.inf
+    got = forward(layer, x, pos, None, lengths, T)
+    keep = np.arange(B) != 3
+    assert np.array_equal(got[keep], clean[keep])
+    err = np.linalg.norm(got[3, :70] - clean[3, :70]) / np.linalg.norm(clean[3, :70])
+    assert err < 2.0 ** -19, err
