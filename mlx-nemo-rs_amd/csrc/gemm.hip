@@ -724,9 +724,12 @@ hipError_t launch_f32_tile(const GemmParams& p, int splits, hipStream_t s) {
 // fp32 activations. The K-parallel kernel has the shorter chain (16 waves
 // share a tile's contraction, 16x16 tiles), the tile kernel the higher rate,
 // so the line is where the K-parallel kernel's work per CU grows past one
-// short tile: 128 tiles of 32x32, 256 where its MFMAs are the same work as
-// the tile kernel's (fp32 weights: three times the products of bf16 ones) or
-// its contraction is short. Measured, us, K-parallel against tile kernel,
+// tile: 256 tiles of 32x32, 224 where the tile kernel takes fewer products
+// (bf16 weights) or the K-parallel kernel dequantises a long contraction.
+// Measured, us, attention steps with a Q/K/V projection of 56 x 3072 x 1024
+// (192 tiles), K-parallel against tile kernel: bf16 26.6 / 31.5, u8 32.3 /
+// 35.4; of 70 x 3072 (288 tiles): bf16 32.7 / 28.1, fp32 weights 32.6 / 30.6,
+// u8 41.1 / 33.6. Single projections, us, K-parallel against tile kernel,
 // K = 1024: fp32 weights 224 x 1024 9.9 / 11.5, 56 x 4096 9.7 / 11.3, 300 x
 // 1024 14.0 / 11.8; u8 112 x 1024 9.9 / 11.5, 56 x 4096 13.5 / 11.9; bf16 112
 // x 1024 7.0 / 8.0, 56 x 4096 9.7 / 8.0; u8 125 x 2048 at K = 512 7.1 / 7.9.
@@ -743,7 +746,7 @@ hipError_t dispatch_f32(const GemmParams& p, hipStream_t s) {
   if (kpar_ok<float>(p)) {
     const int64_t t32 = (int64_t)((p.M + 31) / 32) * (p.N / 32);
     const bool wide = WK == kWF32 || (WK == kWU8 && p.K <= 512);
-    if (t32 <= (wide ? 256 : 128) || !f32_tile_ok(p)) return launch_kpar<WK == kWU8>(p, s);
+    if (t32 <= (wide ? 256 : 224) || !f32_tile_ok(p)) return launch_kpar<WK == kWU8>(p, s);
   }
   if (f32_tile_ok(p)) {
     constexpr int BN = WK == kWBF16 ? 128 : 64, MW = WK == kWBF16 ? 2 : 1, KW = WK == kWBF16 ? 2 : 4;

@@ -9,17 +9,29 @@ enum WKind { kWF32 = 0, kWBF16 = 1, kWU8 = 2 };
 template <int WK>
 __device__ __forceinline__ float f32_dot(const GemmParams& p, int row, int col) {
   const float* a = reinterpret_cast<const float*>(p.A) + (int64_t)row * p.lda;
+  const int64_t w0 = (int64_t)col * p.K;
   float s = 0.f;
+  // (a NaN stays one: rows that hold one end at the group of 64 where it is)
 #pragma unroll 1
-  for (int k = 0; k < p.K; ++k) {
-    float w;
-    if constexpr (WK == kWF32) w = reinterpret_cast<const float*>(p.W)[(int64_t)col * p.K + k];
-    else if constexpr (WK == kWBF16) w = (float)reinterpret_cast<const bf16*>(p.W16)[(int64_t)col * p.K + k];
-    else {
-      const float* sb = p.sb + 2 * ((int64_t)col * (p.K / 64) + k / 64);
-      w = __builtin_fmaf(sb[0], (float)reinterpret_cast<const unsigned char*>(p.W)[(int64_t)col * p.K + k], sb[1]);
+  for (int k0 = 0; k0 < p.K && s == s; k0 += 64) {
+#pragma unroll 4
+    for (int k = k0; k < k0 + 64; k += 4) {
+      const floatx4 av = *reinterpret_cast<const floatx4*>(a + k);
+      floatx4 w;
+      if constexpr (WK == kWF32) {
+        w = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(p.W) + w0 + k);
+      } else if constexpr (WK == kWBF16) {
+        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16*>(p.W16) + w0 + k);
+        w = floatx4{(float)wv[0], (float)wv[1], (float)wv[2], (float)wv[3]};
+      } else {
+        const float* sb = p.sb + 2 * ((int64_t)col * (p.K / 64) + k0 / 64);
+        const uint32_t c = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(p.W) + w0 + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = __builtin_fmaf(sb[0], (float)((c >> (8 * e)) & 0xFFu), sb[1]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = __builtin_fmaf(av[e], w[e], s);
     }
-    s = __builtin_fmaf(a[k], w, s);
   }
   return s;
 }
@@ -323,9 +335,11 @@ __device__ __forceinline__ void f32_tile_body(const GemmParams& p, int splits, i
       for (int s = 0; s < C::KST; ++s) step(kt, s, s & 1);
   }
 
-  if (p.acopy && n0 == 0 && z == 0) {
-    // the first column tile copies its rows of A
-    for (int id = tid; id < (m_end - m0) * (p.K / 4); id += C::NT) {
+  if (p.acopy && z == 0) {
+    // each column tile copies its share of the rows of A (the first tile's
+    // workgroup alone took 3 us longer than the others at 64 x 3072 x 1024)
+    const int total = (m_end - m0) * (p.K / 4), each = (total + tilesN - 1) / tilesN, tn = n0 / BN;
+    for (int id = tn * each + tid; id < min((tn + 1) * each, total); id += C::NT) {
       const int row = m0 + id / (p.K / 4), c = id % (p.K / 4) * 4;
       *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(p.acopy) + mapped_row(p, row) * p.acopy_ld + c) =
           *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(p.A) + (int64_t)row * p.lda + c);
