@@ -367,21 +367,27 @@ __device__ __forceinline__ floatx4 kpar_load(__amdgpu_buffer_rsrc_t r, int voff,
   return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
-template <bool QUANT, int TR>
-__global__ __launch_bounds__(1024) void gemm_kpar_kernel(const GemmParams p) {
+// LDS of a workgroup of up to NW waves: the two reduction buffers [tile
+// parity][wave][element], and TR 1 KB transpose slots per wave
+template <int TR, int NW>
+struct KparSmem {
+  float red[2][NW][256 * TR * TR];
+  char xsm[NW][1024 * TR];
+};
+
+template <bool QUANT, int TR, int NW>
+__device__ __forceinline__ void kpar_body(const GemmParams& p, int block, int G, KparSmem<TR, NW>& sm) {
   // TR x TR blocks of 16x16 per tile: 32x32 tiles (TR = 2), or 16x16 tiles
   // (TR = 1) for problems with too few 32x32 tiles to give each CU one
   constexpr int TS = 16 * TR, EPW = 64 * 4 * TR * TR;  // tile side; partial sums per wave
-  __shared__ __attribute__((aligned(16))) float red[2][16][EPW];  // [tile parity][wave][element]
-  __shared__ __attribute__((aligned(16))) char xsm[16][1024 * TR];  // TR 1 KB transpose slots per wave
   const int tid = threadIdx.x, lane = tid & 63, nt_threads = (int)blockDim.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt_threads >> 6;
-  const int tilesN = p.N / TS, T = (p.M + TS - 1) / TS * tilesN, G = (int)gridDim.x;
-  const int v0 = (int)((int64_t)blockIdx.x * T / G), v1 = (int)((int64_t)(blockIdx.x + 1) * T / G);
+  const int tilesN = p.N / TS, T = (p.M + TS - 1) / TS * tilesN;
+  const int v0 = (int)((int64_t)block * T / G), v1 = (int)((int64_t)(block + 1) * T / G);
   if (v0 >= v1) return;  // (whole workgroup)
   const int kq = w * 64 + 4 * (lane & 3);   // quad-run chunk of the wave's k-columns
   const int kf = w * 64 + 4 * (lane >> 4);  // MFMA-layout chunk
-  char* xs = xsm[w];
+  char* xs = sm.xsm[w];
   const int xw = (lane >> 2) * 64 + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
   const int xr = (lane & 15) * 64 + 16 * ((lane >> 4) ^ ((lane >> 2) & 3));
   // (A rows are addressed from the row tile's first row in the range-checked
@@ -494,7 +500,7 @@ __global__ __launch_bounds__(1024) void gemm_kpar_kernel(const GemmParams p) {
     // element 256 (TR t + u) + 4 l + e of lane l: row 16 t + 4 (l / 16) + e,
     // column 16 u + l % 16 (each 16-byte store of a wave covers 1 KB of
     // consecutive words: no bank conflicts)
-    float (&rb)[16][EPW] = red[v & 1];
+    float (&rb)[NW][EPW] = sm.red[v & 1];
 #pragma unroll
     for (int t = 0; t < TR; ++t)
 #pragma unroll
@@ -518,6 +524,25 @@ __global__ __launch_bounds__(1024) void gemm_kpar_kernel(const GemmParams p) {
     }
     if (v + 1 < v1 && (v + 1) / tilesN != mt_cur) loadA(mt_cur = (v + 1) / tilesN);
   }
+}
+
+template <bool QUANT, int TR>
+__global__ __launch_bounds__(1024) void gemm_kpar_kernel(const GemmParams p) {
+  __shared__ __attribute__((aligned(16))) KparSmem<TR, 16> sm;
+  kpar_body<QUANT, TR, 16>(p, (int)blockIdx.x, (int)gridDim.x, sm);
+}
+
+// Two independent problems of one K <= 512 in one launch (one utterance's
+// Q/K/V and position projections): p1's tiles in workgroups [0, g1), p2's
+// after them. With at most 8 waves a workgroup's LDS leaves room for a second
+// one on its CU, so up to two tiles of 32x32 per CU take one round. (125 x
+// 1536 x 512 with 249 x 512: 7.5 + 5.8 us apart; the layer 27.9 -> 25.5.)
+template <bool QUANT>
+__global__ __launch_bounds__(512) void gemm_kpar_pair_kernel(const GemmParams p1, int g1, const GemmParams p2, int g2) {
+  __shared__ __attribute__((aligned(16))) KparSmem<2, 8> sm;
+  const int block = (int)blockIdx.x;
+  if (block < g1) kpar_body<QUANT, 2, 8>(p1, block, g1, sm);
+  else kpar_body<QUANT, 2, 8>(p2, block - g1, g2, sm);
 }
 
 // Tile side of the K-parallel kernel: 16x16 tiles when 32x32 tiles would
@@ -742,12 +767,15 @@ hipError_t launch_f32_tile(const GemmParams& p, int splits, hipStream_t s) {
 // (K = 4096, N = 1024, fp32 weights: 14 rows 32 -> 10.6 in eight, 224 rows
 // 35 -> 22.6 in four, 700 rows 59 -> 48 in two, the sum pass included).
 template <int WK>
+bool takes_kpar(const GemmParams& p) {
+  if (!kpar_ok<float>(p)) return false;
+  const bool wide = WK == kWF32 || (WK == kWU8 && p.K <= 512);
+  return (int64_t)((p.M + 31) / 32) * (p.N / 32) <= (wide ? 256 : 224) || !f32_tile_ok(p);
+}
+
+template <int WK>
 hipError_t dispatch_f32(const GemmParams& p, hipStream_t s) {
-  if (kpar_ok<float>(p)) {
-    const int64_t t32 = (int64_t)((p.M + 31) / 32) * (p.N / 32);
-    const bool wide = WK == kWF32 || (WK == kWU8 && p.K <= 512);
-    if (t32 <= (wide ? 256 : 224) || !f32_tile_ok(p)) return launch_kpar<WK == kWU8>(p, s);
-  }
+  if (takes_kpar<WK>(p)) return launch_kpar<WK == kWU8>(p, s);
   if (f32_tile_ok(p)) {
     constexpr int BN = WK == kWBF16 ? 128 : 64, MW = WK == kWBF16 ? 2 : 1, KW = WK == kWBF16 ? 2 : 4;
     if (p.N % BN == 0 && (int64_t)((p.M + 63) / 64) * (p.N / BN) >= 512)
@@ -854,8 +882,19 @@ bool gemm_few_tiles(DType dt, bool quantized, const GemmParams& p) {
 // 749 x 1024 position tiles, step 0.064 -> 0.061 ms). Past one round it
 // measured no gain (15000 x 3072 with 257 rows: step 0.2174 against
 // 0.2202 ms). Two problems of few tiles share a launch of gemm_kw_kernel
-// where one round holds both.
+// where one round holds both, and two fp32 ones of the K-parallel kernel.
 namespace {
+// (the waves' sums meet in the same order as alone, in either tile size)
+bool pair_kpar_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
+  if (dt != kF32 || p1.M <= 0 || p2.M <= 0 || p1.K != p2.K || p1.K > 512) return false;
+  int64_t tiles = 0;
+  for (const GemmParams* p : {&p1, &p2}) {
+    if (p->C2 || p->acopy || p->W16 || gemm_check(dt, quantized, *p) != hipSuccess) return false;
+    if (!(quantized ? takes_kpar<kWU8>(*p) : takes_kpar<kWF32>(*p))) return false;
+    tiles += (int64_t)((p->M + 31) / 32) * (p->N / 32);
+  }
+  return tiles <= 2 * device_cus();
+}
 int pair_kw_form(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
   if (!gemm_few_tiles(dt, quantized, p1) || !gemm_few_tiles(dt, quantized, p2)) return 0;
   return quantized ? kw_form<true>(p1, &p2) : kw_form<false>(p1, &p2);
@@ -863,6 +902,7 @@ int pair_kw_form(DType dt, bool quantized, const GemmParams& p1, const GemmParam
 }  // namespace
 
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
+  if (pair_kpar_ok(dt, quantized, p1, p2)) return true;
   if (pair_kw_form(dt, quantized, p1, p2)) return true;
   TileForm f1, f2;
   return gemm_tile_form(dt, quantized, p1, f1) && f1.bm != 64 &&
@@ -874,6 +914,14 @@ bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmPara
 
 hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2, hipStream_t s) {
   if (!gemm_pair_ok(dt, quantized, p1, p2)) return hipErrorInvalidValue;
+  if (dt == kF32) {
+    const int g1 = (p1.M + 31) / 32 * (p1.N / 32), g2 = (p2.M + 31) / 32 * (p2.N / 32);
+    if (quantized)
+      hipLaunchKernelGGL(gemm_kpar_pair_kernel<true>, dim3(g1 + g2), dim3(p1.K), 0, s, p1, g1, p2, g2);
+    else
+      hipLaunchKernelGGL(gemm_kpar_pair_kernel<false>, dim3(g1 + g2), dim3(p1.K), 0, s, p1, g1, p2, g2);
+    return hipGetLastError();
+  }
   if (const int form = pair_kw_form(dt, quantized, p1, p2))
     return quantized ? launch_kw<true>(form, p1, &p2, s) : launch_kw<false>(form, p1, &p2, s);
   TileForm f;

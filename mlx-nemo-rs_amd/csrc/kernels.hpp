@@ -83,10 +83,11 @@ bool gemm_tile_form(DType dt, bool quantized, const GemmParams& p, TileForm& f);
 // Whether gemm() runs this bf16 problem on the kernel for few output tiles
 // (whose sums are in another order than the tile kernels').
 bool gemm_few_tiles(DType dt, bool quantized, const GemmParams& p);
-// Two independent bf16 GEMMs of one weight form in one launch: p2's tiles
-// take the CUs p1's tiles leave. For a p1 that gemm() runs in one round of
+// Two independent GEMMs of one dtype and weight form in one launch: p2's tiles
+// take the CUs p1's tiles leave. For a bf16 p1 that gemm() runs in one round of
 // tiles of a form larger than 64x64 and a p2 it runs in the 64x64 form, and
-// for two of few tiles that together take one round (gemm_pair_ok); the same
+// for two of few tiles that together take one round, in either dtype
+// (gemm_pair_ok); the same
 // results as gemm() on each. Otherwise hipErrorInvalidValue and nothing is
 // launched.
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2);

@@ -112,3 +112,20 @@ def test_scaled_inputs(scale):
     x = (rng.standard_normal((160, 256)) * scale * np.exp2(rng.uniform(-12, 12, size=(160, 256)))).astype(np.float32)
     got = m.debug_linear(0, torch.from_numpy(x).cuda()).cpu().numpy()
     check(got, x.astype(np.float64), dense[0], f"scale {scale}")
+
+
+# one utterance's Q/K/V and position projections in one launch, with 1 to 3
+# row tiles each; the result is that of the two apart
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("d,h,T", [(256, 4, 17), (512, 8, 33), (512, 8, 65)])
+def test_paired_projections(d, h, T, quant):
+    rng = np.random.default_rng(d + T)
+    w = W.make_layer_weights(rng, d, h, not quant, quant, centred=quant)
+    layer = M.RelPositionMultiHeadAttention(d, h, not quant)
+    layer.load_weights(W.prefixed(w, "l"), "l")
+    layer.set_dtype(O.F32)
+    x = torch.from_numpy(rng.standard_normal((1, T, d)).astype(np.float32)).cuda()
+    pos = torch.from_numpy(O.RelPositionalEncoding(d, 5000, True).get_encoding(T)).float().cuda().contiguous()
+    q, P = layer.debug_position_scores(x, pos, with_inputs=True)[1:]
+    assert torch.equal(q, layer.debug_linear("linear_q", x))
+    assert torch.equal(P.reshape(-1, d), layer.debug_linear("linear_pos", pos).reshape(-1, d))
