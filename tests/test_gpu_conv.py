@@ -164,3 +164,30 @@ def test_conv_cache_needs_causal_module():
     with pytest.raises(M.MhsaError) as e:
         m.forward_with_cache(x, cache)
     assert e.value.code == M.MHSA_EINVAL
+
+
+@pytest.mark.parametrize("dtype", [O.F32, O.BF16])
+@pytest.mark.parametrize("kernel,causal", [(9, False), (9, True), (31, False), (32, True), (33, False)])
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 15), (1, 17), (3, 63), (2, 65)])
+def test_frame_tiles_agree(dtype, kernel, causal, B, T):
+    """An item alone or among few takes 16-frame tiles, among enough others
+    64-frame ones: the same values bit for bit, for kernels on both sides of
+    the taps that LDS holds."""
+    d, many = 512, 64
+    rng = np.random.default_rng(kernel + B + T)
+    m = M.ConvolutionModule(d, kernel, "batch_norm", causal, True)
+    w = {"pointwise_conv1.weight": rng.standard_normal((2 * d, d)) / 16, "pointwise_conv1.bias": rng.standard_normal(2 * d),
+         "pointwise_conv2.weight": np.eye(d), "pointwise_conv2.bias": np.zeros(d),
+         "depthwise_conv.weight": rng.standard_normal((d, kernel, 1)) / 3, "depthwise_conv.bias": rng.standard_normal(d),
+         "batch_norm.weight": rng.uniform(0.5, 1.5, d), "batch_norm.bias": rng.standard_normal(d),
+         "batch_norm.running_mean": rng.standard_normal(d), "batch_norm.running_var": rng.uniform(0.5, 2, d)}
+    m.load_weights({"c." + k: v.astype(np.float32) for k, v in w.items()}, "c")
+    m.set_dtype(dtype)
+    # one-hot pointwise_conv1 inputs: each GLU value is one weight and a bias, whatever the GEMM
+    x = torch.zeros((many, T, d), device="cuda", dtype=torch.float32 if dtype == O.F32 else torch.bfloat16)
+    hot = torch.from_numpy(rng.integers(0, d, size=(many, T))).cuda()
+    x.scatter_(2, hot[..., None], 1)
+    lengths = [T] + [max(1, T - 3 * i) for i in range(1, many)]
+    few = m.forward(x[:B].contiguous(), lengths[:B])
+    assert torch.isfinite(few.float()).all()
+    assert torch.equal(few, m.forward(x, lengths)[:B])
