@@ -1429,23 +1429,26 @@ hipError_t launch_ks(const AttnParams& p, int nb, hipStream_t s) {
 template <typename T, int DK>
 hipError_t dispatch_nw(const AttnParams& p, int nb, hipStream_t s) {
   const bool dbg = p.dbg_bd != nullptr;
-  // fp32 inputs too short to give the CUs a workgroup each (one utterance of
-  // 125 frames: 16 workgroups of 64 queries) split their keys over the waves
+  // fp32 inputs of few workgroups of 64 queries (one utterance of 125 frames:
+  // 16) split their keys over the waves of workgroups of 16. Measured, us, a
+  // layer of d_model 1024, key split / 64 queries: 1 x 375 frames (48
+  // workgroups) 97 / 106, 1 x 500 (64) 113 / 126, 2 x 200 (64) 82 / 84, 5 x
+  // 125 (80) 105 / 87, 1 x 700 (88) 205 / 171, 1 x 900 (120) 255 / 210.
   // Short query blocks (the streaming chunk against more keys than the chunk
   // kernel stages) take the key-split form too: a one-wave form of this
   // kernel (16 queries, no split) gave wrong outputs whenever its per-key
   // mask ran, while the key-split form of the same source is exact on those
   // shapes, so there is no one-wave form.
   if constexpr (sizeof(T) == 4) {
-    if (!dbg && (p.T <= 16 || (int64_t)nb * p.H * ((p.T + 63) / 64) < 128))
+    if (!dbg && (p.T <= 16 || (int64_t)nb * p.H * ((p.T + 63) / 64) <= 64))
       return launch_ks<T, DK, 4>(p, nb, s);  // (per-wave tiles: 34 / 37 KB of LDS)
-    if (!dbg) {
-      hipLaunchKernelGGL((attn_f32_kernel<DK>), dim3(p.H, (p.T + 63) / 64, nb), dim3(256), 0, s, p);
-      count_form(kFormGeneric);
-      return hipGetLastError();
-    }
+    if (dbg) return launch<T, DK, 4, true>(p, nb, s);
+    hipLaunchKernelGGL((attn_f32_kernel<DK>), dim3(p.H, (p.T + 63) / 64, nb), dim3(256), 0, s, p);
+    count_form(kFormGeneric);
+    return hipGetLastError();
+  } else {
+    return dbg ? launch<T, DK, 4, true>(p, nb, s) : launch<T, DK, 4, false>(p, nb, s);
   }
-  return dbg ? launch<T, DK, 4, true>(p, nb, s) : launch<T, DK, 4, false>(p, nb, s);
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
