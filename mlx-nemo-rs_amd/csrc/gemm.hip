@@ -16,9 +16,11 @@
 //    one short utterance): persistent workgroups over 32 x 32 tiles, each
 //    tile's contraction split over the K / 64 waves of a workgroup and summed
 //    in LDS.
-//  * gemm_kw_kernel: bf16 projections of few output tiles (one utterance, a
-//    short position table), the contraction shared by the waves of a
-//    workgroup (gemm_kw_tile.hpp).
+//  * gemm_chain_kernel: bf16 projections of few output tiles (one utterance, a
+//    short position table), each sum the tile kernel's chain, loads and
+//    dequantisation by waves of their own (gemm_chain_tile.hpp).
+//  * gemm_kw_kernel: bf16 projections of fewer still, whose sums are those of
+//    runs of the contraction, a wave each (gemm_kw_tile.hpp).
 //  * gemm_kernel: everything else (shapes and alignments the others do not
 //    take): BM x BN tiles on NWM x NWN waves, one 128-byte K step per LDS
 //    stage, double-buffered with a 16-byte row pad; an optional deterministic
@@ -42,6 +44,7 @@ constexpr int PITCH = ROWB + 16;  // LDS row pitch (bytes)
 
 #include "gemm_tile.hpp"
 #include "gemm_f32_tile.hpp"
+#include "gemm_chain_tile.hpp"
 #include "gemm_kw_tile.hpp"
 
 template <typename T, bool QUANT, int BN, int NT>
@@ -623,9 +626,10 @@ bool tile_ok(const GemmParams& p) {
   return true;
 }
 
-// bf16 projections past kw_form's line go to the tile kernel: with at least
-// ~100 tiles of 128 x 128 at the tile shape with the lowest estimated time,
-// below that as 64 x 64 tiles with four stages.
+// bf16 projections of at least 16 tiles of 64 x 64 are the tile kernel's:
+// with at least ~100 tiles of 128 x 128 at the tile shape with the lowest
+// estimated time, below that as 64 x 64 tiles with four stages (or, past
+// which chain_form draws a line, as gemm_chain_kernel, the same sums).
 // Stages: three (loads two ahead) for 192 x 192, 192 x 128 and the u8
 // 192 x 256; four for a 128 x 128 tile that has its CU to itself, two when
 // two share one; 256 x 256 and the dense 192 x 256 fit two. Returns false
@@ -633,6 +637,7 @@ bool tile_ok(const GemmParams& p) {
 bool tile_form(const GemmParams& p, TileForm& f) {
   if (!tile_ok(p) || p.N % 64) return false;
   if (p.N % 128 || m_tiles<128>(p) * (p.N / 128) < 96) {
+    if (m_tiles<64>(p) * (p.N / 64) < 16) return false;
     f = TileForm{64, 64, 4};
     return true;
   }
@@ -659,26 +664,38 @@ bool dispatch_tile(const GemmParams& p, hipStream_t s, hipError_t& err) {
   return true;
 }
 
-// Form of gemm_kw_kernel for one problem, or for two in one launch: 32 x 32
+// Fewer than 16 tiles of 64 x 64: the sums are those of runs of 256 k-columns
+// (gemm_kw_kernel) where K is whole runs. (The tile form of such a problem, a
+// few workgroups in one chain each, measured slower, and its sums are others,
+// so the line is not moved with the kernels' speed.)
+bool kw_ok(const GemmParams& p) {
+  return tile_ok(p) && !p.vt && p.N % 64 == 0 && p.K % 256 == 0 && m_tiles<64>(p) * (p.N / 64) < 16;
+}
+
+template <bool QUANT>
+hipError_t launch_kw(const GemmParams& p, hipStream_t s) {
+  hipLaunchKernelGGL(gemm_kw_kernel<QUANT>, dim3((unsigned)((p.M + 31) / 32 * (p.N / 32))), dim3(512), 0, s, p);
+  return hipGetLastError();
+}
+
+// Form of gemm_chain_kernel for one problem, or for two in one launch: 32 x 32
 // tiles, 64 x 32 or 64 x 64, the smallest that gives no CU a second tile (a
 // workgroup's LDS has the CU to itself, so a second round costs as much as
-// the first), 0 if none does. The forms sum in the same order. Measured, us a launch, 32 x 32 / 64 x 32 /
-// 64 x 64 against the 64 x 64 tile kernel:
-//   u8    125 x 1024 x 1024   4.4 /  5.0 /  6.8 against  8.6
-//         125 x 4096 x 1024   7.6 /  5.2 /  7.0 against  9.1
-//         203 x 4096 x 1024  13.0 /  8.9 /  7.2 against  9.7
-//         203 x 1024 x 4096   9.1 / 10.2 / 15.2 against 24.3
-//         700 x 1024 x 4096  24.2 / 22.3 / 17.8 against 25.5
-//   bf16  125 x 1024 x 1024   4.1 /  4.9 /  6.4 against  5.8
-//         400 x 1024 x 4096  14.5 / 10.6 / 14.4 against 15.0
-//         203 x 4096 x 1024  12.5 /  8.9 /  7.2 against  6.7
-// so one dense problem does not take the 64 x 64 form (the tile kernel's
-// four waves are as fast where nothing is dequantised), but a pair does: it
-// saves a launch of 4 us.
+// the first), 0 if none does or the problem is no tile kernel's. The sums are
+// the tile kernel's. Measured, us a launch, 64 x 64 tile kernel / this:
+//   32 x 32  bf16   1 x 4096 x 1024   6.2 / 5.5,  203 x 1024 x 4096  14.7 / 9.0
+//            u8   203 x 1024 x 4096  23.9 / 12.0, 400 x 512 x 2048   14.1 / 8.2
+//   64 x 32  bf16 400 x 1024 x 4096  15.9 / 11.6, 125 x 4096 x 1024   7.6 / 7.4
+//            u8   400 x 1024 x 4096  24.5 / 13.7, 125 x 4096 x 1024  10.3 / 7.6
+//   64 x 64  u8   700 x 1024 x 4096  25.1 / 19.6, 203 x 4096 x 1024  11.4 / 10.3
+// One dense problem does not take the 64 x 64 form (the tile kernel's four
+// waves are as fast where nothing is dequantised), but a pair does: it saves a
+// launch of 4 us.
 template <bool QUANT>
-int kw_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
-  if (p1.one_chain || !tile_ok(p1) || p1.N % 64) return 0;
+int chain_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
   const int64_t cus = device_cus();
+  for (const GemmParams* p : {&p1, p2})
+    if (p && (!tile_ok(*p) || p->N % 64 || m_tiles<64>(*p) * (p->N / 64) < 16)) return 0;
   auto tiles = [&](auto count) { return count(p1) + (p2 ? count(*p2) : 0); };
   if (tiles([](const GemmParams& p) { return m_tiles<32>(p) * (p.N / 32); }) <= cus) return 1;
   if (tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 32); }) <= cus) return 2;
@@ -686,18 +703,20 @@ int kw_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
   return 0;
 }
 
+template <int TM, int TN, int R, bool QUANT>
+hipError_t launch_chain_tile(const GemmParams& p1, const GemmParams* p2, hipStream_t s) {
+  auto blocks = [](const GemmParams& p) { return (int)((m_tiles<32 * TM>(p) * (p.N / (32 * TN)) + 7) / 8 * 8); };
+  const int n1 = blocks(p1), n2 = p2 ? blocks(*p2) : 0;
+  hipLaunchKernelGGL((gemm_chain_kernel<TM, TN, R, QUANT>), dim3((unsigned)(n1 + n2)),
+                     dim3(ChainTile<TM, TN, R, QUANT>::NT), 0, s, p1, n1, p2 ? *p2 : p1);
+  return hipGetLastError();
+}
+
 template <bool QUANT>
-hipError_t launch_kw(int form, const GemmParams& p1, const GemmParams* p2, hipStream_t s) {
-  auto go = [&](auto kernel, int64_t t1, int64_t t2) {
-    const int n1 = (int)((t1 + 7) / 8 * 8), n2 = (int)((t2 + 7) / 8 * 8);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(n1 + n2)), dim3(512), 0, s, p1, n1, p2 ? *p2 : p1);
-    return hipGetLastError();
-  };
-  if (form == 1)
-    return go(gemm_kw_kernel<1, 1, 8, 2, QUANT>, m_tiles<32>(p1) * (p1.N / 32), p2 ? m_tiles<32>(*p2) * (p2->N / 32) : 0);
-  if (form == 2)
-    return go(gemm_kw_kernel<2, 1, 8, 1, QUANT>, m_tiles<64>(p1) * (p1.N / 32), p2 ? m_tiles<64>(*p2) * (p2->N / 32) : 0);
-  return go(gemm_kw_kernel<2, 2, 8, 1, QUANT>, m_tiles<64>(p1) * (p1.N / 64), p2 ? m_tiles<64>(*p2) * (p2->N / 64) : 0);
+hipError_t launch_chain(int form, const GemmParams& p1, const GemmParams* p2, hipStream_t s) {
+  if (form == 1) return launch_chain_tile<1, 1, QUANT ? 5 : 4, QUANT>(p1, p2, s);
+  if (form == 2) return launch_chain_tile<2, 1, 3, QUANT>(p1, p2, s);
+  return launch_chain_tile<2, 2, QUANT ? 5 : 4, QUANT>(p1, p2, s);
 }
 
 template <typename T, bool QUANT, int BM, int BN, int NWM, int NWN>
@@ -795,7 +814,8 @@ template <bool QUANT>
 hipError_t dispatch_bf16(const GemmParams& p, hipStream_t s) {
   using T = bf16;
   hipError_t err;
-  if (const int form = kw_form<QUANT>(p)) return launch_kw<QUANT>(form, p, nullptr, s);
+  if (kw_ok(p)) return launch_kw<QUANT>(p, s);
+  if (const int form = chain_form<QUANT>(p)) return launch_chain<QUANT>(form, p, nullptr, s);
   if (dispatch_tile<QUANT>(p, s, err)) return err;
   // 256x256 (8 waves) when it still fills the GPU about twice over: it
   // halves the LDS and L2 traffic per flop of 128x128 (measured 1.15x on
@@ -835,8 +855,7 @@ hipError_t gemm_check(DType dt, bool quantized, const GemmParams& p) {
 }
 
 bool gemm_tile_form(DType dt, bool quantized, const GemmParams& p, TileForm& f) {
-  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess &&
-         !gemm_few_tiles(dt, quantized, p) && tile_form(p, f);
+  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess && tile_form(p, f);
 }
 
 namespace {
@@ -872,16 +891,11 @@ int device_cus() {
   return n;
 }
 
-bool gemm_few_tiles(DType dt, bool quantized, const GemmParams& p) {
-  return dt == kBF16 && p.M > 0 && !p.C2 && !p.acopy && gemm_check(dt, quantized, p) == hipSuccess &&
-         (quantized ? kw_form<true>(p) : kw_form<false>(p));
-}
-
 // Paired where p1's tiles take one round of CUs: the CUs its slowest tiles
 // leave idle then run p2's tiles (measured: 3000 x 3072 Q/K/V tiles with
 // 749 x 1024 position tiles, step 0.064 -> 0.061 ms). Past one round it
 // measured no gain (15000 x 3072 with 257 rows: step 0.2174 against
-// 0.2202 ms). Two problems of few tiles share a launch of gemm_kw_kernel
+// 0.2202 ms). Two problems of few tiles share a launch of gemm_chain_kernel
 // where one round holds both, and two fp32 ones of the K-parallel kernel.
 namespace {
 // (the waves' sums meet in the same order as alone, in either tile size)
@@ -895,15 +909,16 @@ bool pair_kpar_ok(DType dt, bool quantized, const GemmParams& p1, const GemmPara
   }
   return tiles <= 2 * device_cus();
 }
-int pair_kw_form(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
-  if (!gemm_few_tiles(dt, quantized, p1) || !gemm_few_tiles(dt, quantized, p2)) return 0;
-  return quantized ? kw_form<true>(p1, &p2) : kw_form<false>(p1, &p2);
+int pair_chain_form(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
+  for (const GemmParams* p : {&p1, &p2})
+    if (dt != kBF16 || p->M <= 0 || p->C2 || p->acopy || gemm_check(dt, quantized, *p) != hipSuccess) return 0;
+  return quantized ? chain_form<true>(p1, &p2) : chain_form<false>(p1, &p2);
 }
 }  // namespace
 
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2) {
   if (pair_kpar_ok(dt, quantized, p1, p2)) return true;
-  if (pair_kw_form(dt, quantized, p1, p2)) return true;
+  if (pair_chain_form(dt, quantized, p1, p2)) return true;
   TileForm f1, f2;
   return gemm_tile_form(dt, quantized, p1, f1) && f1.bm != 64 &&
          gemm_tile_form(dt, quantized, p2, f2) && f2.bm == 64 &&
@@ -922,8 +937,8 @@ hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmP
       hipLaunchKernelGGL(gemm_kpar_pair_kernel<false>, dim3(g1 + g2), dim3(p1.K), 0, s, p1, g1, p2, g2);
     return hipGetLastError();
   }
-  if (const int form = pair_kw_form(dt, quantized, p1, p2))
-    return quantized ? launch_kw<true>(form, p1, &p2, s) : launch_kw<false>(form, p1, &p2, s);
+  if (const int form = pair_chain_form(dt, quantized, p1, p2))
+    return quantized ? launch_chain<true>(form, p1, &p2, s) : launch_chain<false>(form, p1, &p2, s);
   TileForm f;
   tile_form(p1, f);
   return quantized ? dispatch_pair<true>(f, p1, p2, s) : dispatch_pair<false>(f, p1, p2, s);

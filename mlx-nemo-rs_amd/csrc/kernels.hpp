@@ -62,10 +62,6 @@ struct GemmParams {
   // half-step residual R + 0.5 y; exact in either dtype)
   int act = 0;
   float res_scale = 1.f;
-  // bf16: each sum is one chain along K, as in the tile kernels, so position
-  // rows that a stream projects once and keeps, or that are projected alone
-  // to compare, are those of a long input's position tiles bit for bit
-  bool one_chain = false;
 };
 constexpr int kActSilu = 1;
 // Scratch the K-split path can use: 64x64 tiles x splits stays <= ~512
@@ -74,22 +70,18 @@ constexpr int64_t kGemmPartialElems = (int64_t)1 << 22;
 hipError_t gemm(DType dt, bool quantized, const GemmParams& p, hipStream_t s);
 // gemm()'s argument checks alone (p.M > 0 assumed).
 hipError_t gemm_check(DType dt, bool quantized, const GemmParams& p);
-// The tile GEMM form (tile rows, tile columns, LDS stages) gemm() launches
-// for a valid bf16 problem; false when it takes another kernel.
+// The tile GEMM form (tile rows, tile columns, LDS stages) whose sums gemm()
+// gives for a valid bf16 problem; false when another kernel's are.
 struct TileForm {
   int bm = 0, bn = 0, ns = 0;
 };
 bool gemm_tile_form(DType dt, bool quantized, const GemmParams& p, TileForm& f);
-// Whether gemm() runs this bf16 problem on the kernel for few output tiles
-// (whose sums are in another order than the tile kernels').
-bool gemm_few_tiles(DType dt, bool quantized, const GemmParams& p);
 // Two independent GEMMs of one dtype and weight form in one launch: p2's tiles
 // take the CUs p1's tiles leave. For a bf16 p1 that gemm() runs in one round of
-// tiles of a form larger than 64x64 and a p2 it runs in the 64x64 form, and
-// for two of few tiles that together take one round, in either dtype
-// (gemm_pair_ok); the same
-// results as gemm() on each. Otherwise hipErrorInvalidValue and nothing is
-// launched.
+// tiles of a form larger than 64x64 and a p2 of the 64x64 form, and for two of
+// few tiles that together take one round, in either dtype (gemm_pair_ok); the
+// same results as gemm() on each. Otherwise hipErrorInvalidValue and nothing
+// is launched.
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2);
 hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2, hipStream_t s);
 // Whether gemm() takes this problem with C2 / acopy set (fp32, few rows).

@@ -243,16 +243,6 @@ int32_t run_gemm(mhsa_layer* L, DType dt, const DevLinear& lin, int n_rows_w, co
   return MHSA_OK;
 }
 
-// The position rows in the layer dtype, apart from an offline forward (the
-// streaming memo and the debug entry): one_chain's sums.
-int32_t pos_rows_alone(mhsa_layer* L, const void* pos_emb, int rows, void* out, hipStream_t s) {
-  mhsa::GemmParams g;
-  if (int32_t rc = make_gemm(L, L->dev[4], L->D, pos_emb, L->D, rows, out, L->D, nullptr, 0, g)) return rc;
-  g.one_chain = true;
-  HIPCHK(mhsa::gemm(L->dt, L->dev[4].quantized, g, s));
-  return MHSA_OK;
-}
-
 // q, k, v (and optionally only k, v) projections of `A` [M, D].
 // With `vt`, V goes to the transposed buffer instead of columns [2D, 3D).
 int32_t project_qkv(mhsa_layer* L, const void* A, int M, void* out, int64_t ldo, hipStream_t s,
@@ -393,7 +383,6 @@ struct OfflineLayout {
   int row0 = 0, nrows = 0, center = 0, pad = 0, kv_pad = 0;
   int64_t M = 0;
   bool use_vt = false;
-  bool few = false;    // the Q/K/V projection is one of few tiles
   char* qkv = nullptr;
   char* P = nullptr;   // table rows [0, nrows) after `pad` slack rows
   char* cx = nullptr;
@@ -471,25 +460,13 @@ int32_t offline_layout(mhsa_layer* L, int B, int T, int pos_len, const mhsa_cont
   }
   o.P = o.qkv + qkv_b + (size_t)o.pad * D * es;
   o.cx = o.qkv + qkv_b + p_b;
-  if (L->qkv_fused && o.use_vt) {
-    VtOut v = o.vt;
-    v.col0 = 2 * D;
-    mhsa::GemmParams g;  // (o.qkv stands for x, which is 16-byte aligned too)
-    if ((rc = make_gemm(L, L->dev[0], 3 * D, o.qkv, D, (int)o.M, o.qkv, 3 * D, nullptr, 0, g, 0, 0, 0, 0, &v))) return rc;
-    o.few = mhsa::gemm_few_tiles(L->dt, L->dev[0].quantized, g);
-  }
   return MHSA_OK;
 }
 
 // The position projection P = pos_emb[row0 : row0 + nrows] W_pos^T of a layout.
-// Its sums' order follows the Q/K/V projection's, whether the two share a
-// launch or not, so a stack gives its layers' results one by one.
 int32_t pos_gemm(mhsa_layer* L, const OfflineLayout& o, const void* pos_emb, mhsa::GemmParams& g) {
-  if (int32_t rc = make_gemm(L, L->dev[4], L->D, static_cast<const char*>(pos_emb) + (size_t)o.row0 * L->D * esz(L),
-                             L->D, o.nrows, o.P, L->D, nullptr, 0, g))
-    return rc;
-  g.one_chain = !o.few;
-  return MHSA_OK;
+  return make_gemm(L, L->dev[4], L->D, static_cast<const char*>(pos_emb) + (size_t)o.row0 * L->D * esz(L), L->D,
+                   o.nrows, o.P, L->D, nullptr, 0, g);
 }
 
 // A projection to launch together with this call's attention (the next
@@ -1123,7 +1100,8 @@ int32_t stream_step(mhsa_layer* L, mhsa_stream* S, const void* x, int B, int T, 
     LayerProf ps(L, "gemm_pos", s, true, false);
     if (L->dt == mhsa::kBF16) {
       HIPCHK(L->pmemo_bf16.ensure(align_up((int64_t)pos_len * D * 2, 256)));
-      if ((rc = pos_rows_alone(L, pos_emb, pos_len, L->pmemo_bf16.p, s))) return rc;
+      if ((rc = run_gemm(L, mhsa::kBF16, L->dev[4], D, pos_emb, D, pos_len, L->pmemo_bf16.p, D, nullptr, 0, s)))
+        return rc;
       HIPCHK(mhsa::widen_bf16(L->pmemo_bf16.p, static_cast<float*>(L->pmemo.p), (int64_t)pos_len * D, s));
     } else if ((rc = run_gemm(L, mhsa::kF32, L->sdev[4], D, pos_emb, D, pos_len, L->pmemo.p, D, nullptr, 0, s))) {
       return rc;
@@ -1473,9 +1451,7 @@ int32_t mhsa_debug_linear(mhsa_layer* L, int32_t which, const void* x, int32_t r
   int32_t rc = prepare(L);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(hs);
-  rc = which == 4 ? pos_rows_alone(L, x, rows, out, s)
-                  : run_gemm(L, L->dt, L->dev[which], L->D, x, L->D, rows, out, L->D, nullptr, 0, s);
-  if (rc) return rc;
+  if ((rc = run_gemm(L, L->dt, L->dev[which], L->D, x, L->D, rows, out, L->D, nullptr, 0, s))) return rc;
   HIPCHK(hipStreamSynchronize(s));
   return MHSA_OK;
 }

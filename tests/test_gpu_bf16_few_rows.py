@@ -1,7 +1,8 @@
-"""The bf16 projections of few output tiles, whose contraction the waves of a
-workgroup share: remainders of the row tiles, waves without a stage, uneven
-stages, each tile form on both sides of its line, and V^T of an utterance
-that ends inside an attention tile.
+"""The bf16 projections of few output tiles: remainders of the row tiles, waves
+without a stage, uneven stages, each tile form on both sides of its line, V^T
+of an utterance that ends inside an attention tile, and the order of their
+sums, which is that of the large tiles or, for a handful of tiles, of runs of
+256 columns.
 
 A result is the bf16 rounding of an fp32 sum: 2^-8 of the value (half a unit
 in the last place at most) and K 2^-24 |A| |W|^T for the sum's roundings.
@@ -61,6 +62,50 @@ def test_linears(d, f, rows, quant):
         x = x.astype(np.float64)
         ref, mag = x @ dense[i].T, np.abs(x) @ np.abs(dense[i]).T
         assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 1.01 * k * 2.0 ** -24 * mag).all(), f"linear{i + 1}"
+
+
+# K of 1 to 64 stages (phases of four or two, ends inside one), and every tile
+# form: 32 x 32 up to 256 rows of 1024 columns, 64 x 32 up to 512, 64 x 64
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("k,rows", [(64, 40), (128, 33), (192, 1), (256, 64), (320, 31), (384, 257), (448, 65), (512, 500),
+                                    (576, 129), (704, 400), (1024, 203), (1024, 700), (1344, 300), (2240, 97),
+                                    (4096, 203), (4096, 400), (4096, 641)])
+def test_rows_alone_and_in_a_batch(k, rows, quant):
+    """Rows give the same results bit for bit alone and among enough others
+    for the large tiles."""
+    rng = np.random.default_rng(k + rows)
+    part, _ = linear(rng, 1024, k, quant)
+    ff = M.FeedForward(k, 1024, False)
+    w = {"f.linear1.%s" % n: v for n, v in part.items()}
+    w.update({"f.linear2.%s" % n: v for n, v in linear(rng, k, 1024, quant)[0].items()})
+    ff.load_weights(w, "f")
+    ff.set_dtype(O.BF16)
+    x = torch.from_numpy(rng.standard_normal((1600, k)).astype(np.float32)).cuda().bfloat16()
+    assert torch.equal(ff.debug_linear(0, x[:rows].contiguous()), ff.debug_linear(0, x)[:rows])
+
+
+# 8 runs are one round of the waves, 9 and 17 two and three
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("f,rows", [(768, 1), (2048, 33), (2304, 64), (4352, 31)])
+def test_runs_of_the_contraction(f, rows, quant):
+    """Fewer than 16 tiles: 2^24 in the first run and -2^24 in the last leave
+    what the runs between add up to, 1 + 1 from two steps of one run, which a
+    single chain would lose one by one."""
+    d = 64
+    m, x = np.zeros((d, f), dtype=np.float32), np.zeros((rows, f), dtype=np.float32)
+    for k, a, b in ((0, 4096, 4096), (256, 1, 1), (320, 1, 1), (f - 1, 4096, -4096)):
+        m[:, k], x[:, k] = a, b
+    w = {"f.linear1.weight": np.zeros((f, d), dtype=np.float32), "f.linear2.weight": m}
+    if quant:
+        sc = np.ones((d, f // 64), dtype=np.float16)
+        sc[:, 0] = sc[:, -1] = 4096
+        w.update({"f.linear2.weight": W.pack_u8((m != 0).astype(np.int64)), "f.linear2.scales": sc,
+                  "f.linear2.biases": np.zeros_like(sc)})
+    ff = M.FeedForward(d, f, False)
+    ff.load_weights(w, "f", M.QuantizationConfig() if quant else None)
+    ff.set_dtype(O.BF16)
+    got = ff.debug_linear(1, torch.from_numpy(x).cuda().bfloat16()).float().cpu().numpy()
+    assert (got == 2.0).all(), np.unique(got)
 
 
 # Q/K/V with V^T and the position rows, in one launch or apart
