@@ -21,8 +21,8 @@
 //    dequantisation by waves of their own (gemm_chain_tile.hpp).
 //  * gemm_kw_kernel: bf16 projections of fewer still, whose sums are those of
 //    runs of the contraction, a wave each (gemm_kw_tile.hpp).
-//  * gemm_kernel: everything else (shapes and alignments the others do not
-//    take): BM x BN tiles on NWM x NWN waves, one 128-byte K step per LDS
+//  * gemm_kernel: everything else (bf16 projections of K without runs of 256,
+//    operands past 2 GiB, alignments that no entry point gives): BM x BN tiles on NWM x NWN waves, one 128-byte K step per LDS
 //    stage, double-buffered with a 16-byte row pad; an optional deterministic
 //    K split with gemm_reduce.
 //
@@ -743,14 +743,14 @@ int small_splits(const GemmParams& p) {
   return splits;
 }
 
-// The fp32 tile kernel's operands: 16-byte rows addressable by 32-bit buffer
-// offsets.
+// The fp32 tile kernel's operands: 16-byte rows, a tile's of which (up to 64 of
+// A, 128 of W) are addressable by 32-bit buffer offsets.
 bool f32_tile_ok(const GemmParams& p) {
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   if (p.vt || p.seg_T || p.K % 64 || p.N % 64 || p.lda % 4 || p.ldc % 4 || (p.R && p.ldr % 4)) return false;
   if (!a16(p.A) || !a16(p.W) || !a16(p.W16) || !a16(p.C) || !a16(p.R) || !a16(p.bias) || !a16(p.sb)) return false;
   if (p.C2 && (!a16(p.C2) || p.ldc2 % 4 || p.c2_col0 % 4)) return false;
-  return (int64_t)p.M * p.lda * 4 < ((int64_t)1 << 31) && (int64_t)p.N * p.K * 4 < ((int64_t)1 << 31);
+  return 64 * p.lda * 4 < ((int64_t)1 << 31) && 128 * (int64_t)p.K * 4 < ((int64_t)1 << 31);
 }
 
 template <int BM, int BN, int MW, int NW, int KW, int WK>
@@ -806,7 +806,7 @@ hipError_t dispatch_f32(const GemmParams& p, hipStream_t s) {
       splits *= 2;
     return launch_f32_tile<32, 64, 1, 1, 4, WK>(p, splits, s);
   }
-  // operands that are not in 16-byte rows
+  // contractions of 4 M columns or more
   return launch<float, WK == kWU8, 64, 64, 2, 2>(p, small_splits<float>(p), s);
 }
 

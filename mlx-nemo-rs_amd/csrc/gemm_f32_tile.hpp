@@ -135,9 +135,10 @@ __device__ __forceinline__ void f32_tile_body(const GemmParams& p, int splits, i
   // lane l stores row l / 16, 16-byte chunk l % 16, which holds chunk
   // (l % 16) ^ (row % 16), so the 16 rows an LDS read serves together hit
   // all 64 banks. bf16 and u8 rows as in the bf16 tile kernel.
+  // (the tile's rows alone: all of A may be past 2 GiB)
   const char* Ab = reinterpret_cast<const char*>(p.A) + (int64_t)m0 * p.lda * 4;
   const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, (int)((int64_t)(p.M - m0) * p.lda * 4), kRawBuffer);
+      __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, (int)((int64_t)(m_end - m0) * p.lda * 4), kRawBuffer);
   int aoff[C::NA], boff[C::NB];
 #pragma unroll
   for (int g = 0; g < C::NA; ++g) {

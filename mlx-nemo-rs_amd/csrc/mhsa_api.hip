@@ -1162,16 +1162,11 @@ int32_t stream_step(mhsa_layer* L, mhsa_stream* S, const void* x, int B, int T, 
     } else {
       if ((rc = run_gemm(L, mhsa::kF32, L->sdev[0], D, x, D, (int)M, q, D, nullptr, 0, s))) return rc;
       ps_kv.next("gemm_kv", false);
-      if (L->qkv_fused) {
-        if ((rc = run_gemm(L, mhsa::kF32, L->sdev[1], 2 * D, x, D, (int)M, kv, 2 * D, nullptr, 0, s, T, R, slot, R)))
-          return rc;
-      } else {
-        if ((rc = run_gemm(L, mhsa::kF32, L->sdev[1], D, x, D, (int)M, kv, 2 * D, nullptr, 0, s, T, R, slot, R)))
-          return rc;
-        if ((rc = run_gemm(L, mhsa::kF32, L->sdev[2], D, x, D, (int)M, kv + (size_t)D * 4, 2 * D, nullptr, 0, s, T,
-                           R, slot, R)))
-          return rc;
-      }
+      if ((rc = run_gemm(L, mhsa::kF32, L->sdev[1], D, x, D, (int)M, kv, 2 * D, nullptr, 0, s, T, R, slot, R)))
+        return rc;
+      if ((rc = run_gemm(L, mhsa::kF32, L->sdev[2], D, x, D, (int)M, kv + (size_t)D * 4, 2 * D, nullptr, 0, s, T,
+                         R, slot, R)))
+        return rc;
       ps_kv.next("ring_write", false);
       HIPCHK(mhsa::ring_write(mhsa::kF32, x, S->ring_h.p, B, T, D, R, D, slot, s));
     }

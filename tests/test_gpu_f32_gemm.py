@@ -80,6 +80,19 @@ def test_linear2_splits(d, f, rows, kind):
     check(got, x.astype(np.float64), dense[1], f"linear2 {kind} {rows}x{d}x{f}")
 
 
+def test_rows_past_two_gib():
+    """131,137 rows of 4096: the activations' last rows lie past 2^31 bytes,
+    and give bit for bit what the same rows give among 33,000."""
+    rng = np.random.default_rng(3)
+    m, _ = make_ff(rng, 64, 4096, "f32")
+    few = torch.randn((33000, 4096), generator=torch.Generator("cuda").manual_seed(3), device="cuda")
+    x = torch.zeros((131137, 4096), device="cuda")
+    x[-33000:] = few
+    got = m.debug_linear(1, x)
+    assert torch.equal(got[-33000:], m.debug_linear(1, few))
+    assert not got[:-33000].any()
+
+
 @pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
 @pytest.mark.parametrize("which,rows", [(0, 130), (1, 40)])
 def test_values_that_are_not_finite(which, rows, kind):
