@@ -771,12 +771,13 @@ hipError_t launch_f32_tile(const GemmParams& p, int splits, hipStream_t s) {
 // tile: 256 tiles of 32x32, 224 where the tile kernel takes fewer products
 // (bf16 weights) or the K-parallel kernel dequantises a long contraction.
 // Measured, us, attention steps with a Q/K/V projection of 56 x 3072 x 1024
-// (192 tiles), K-parallel against tile kernel: bf16 26.6 / 31.5, u8 32.3 /
-// 35.4; of 70 x 3072 (288 tiles): bf16 32.7 / 28.1, fp32 weights 32.6 / 30.6,
-// u8 41.1 / 33.6. Single projections, us, K-parallel against tile kernel,
-// K = 1024: fp32 weights 224 x 1024 9.9 / 11.5, 56 x 4096 9.7 / 11.3, 300 x
-// 1024 14.0 / 11.8; u8 112 x 1024 9.9 / 11.5, 56 x 4096 13.5 / 11.9; bf16 112
-// x 1024 7.0 / 8.0, 56 x 4096 9.7 / 8.0; u8 125 x 2048 at K = 512 7.1 / 7.9.
+// (192 tiles), K-parallel against tile kernel: bf16 26.6 / 31.5; of 70 x 3072
+// (288 tiles): bf16 32.7 / 28.1. Single projections, us, K-parallel against
+// tile kernel, K = 1024: fp32 weights 224 x 1024 10.1 / 12.8, 56 x 4096 12.2 /
+// 14.0, 300 x 1024 15.0 / 13.4, 65 x 3072 15.2 / 13.8; u8 112 x 1024 11.6 /
+// 12.6, 224 x 1024 13.6 / 13.0, 56 x 4096 14.8 / 13.8, 65 x 3072 20.6 / 13.7;
+// bf16 112 x 1024 7.0 / 8.0, 56 x 4096 9.7 / 8.0; u8 125 x 2048 at K = 512
+// 8.6 / 10.3.
 //
 // Tile: the large one (64 x 128 for bf16 weights, 64 x 64 else) from 512
 // tiles, two per CU, on; 32 x 64 below (1500 x 4096 x 1024: bf16 44 / 54,

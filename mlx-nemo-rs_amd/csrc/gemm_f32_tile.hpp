@@ -65,7 +65,7 @@ __device__ __forceinline__ void f32_store(const GemmParams& p, int row, int col,
 // fp32 activations times fp32, bf16 or u8 weights. The fp32 MFMA is what
 // bounded the kernels before (157 TFLOP/s, a sixteenth of the bf16 one), so
 // the operands go through the bf16 MFMAs in three exact parts: three products
-// per weight that is a bf16 value, six per fp32 or dequantised one. Operands
+// per weight that is a bf16 value, eight per fp32 or dequantised one. Operands
 // stream raw through NS LDS stages of 64 k-columns with direct-to-LDS loads
 // (fp32 rows are 4 bytes a value there against 6 for their parts), and each
 // wave splits its fragments in registers, one step ahead, between the MFMAs
@@ -75,11 +75,13 @@ __device__ __forceinline__ void f32_store(const GemmParams& p, int row, int col,
 // where no fragment is split twice, and along M only with bf16 weights, which
 // need no split; two workgroups per CU overlap each other's barriers.
 // Measured (us before / now, MFMA rate now in bf16 products), 1500 rows:
-// 4096 x 1024 bf16 weights 154 / 44 (860 TFLOP/s), fp32 155 / 85 (890), u8
-// 157 / 88; 1024 x 4096 bf16 169 / 48, fp32 171 / 94; 224 rows: 4096 x 1024
-// bf16 25.5 / 10.8, fp32 25.8 / 19.4, 1024 x 4096 bf16 30.5 / 15.0, fp32 30.6
-// / 22.6. Its error against 64 bits is 0.9-1.3e-7 at K = 1024 (K-parallel
-// kernel 1.6-1.8e-7, fp32 tiles before 5.3-6.4e-7).
+// 4096 x 1024 bf16 weights 154 / 44 (860 TFLOP/s), fp32 155 / 108 (930), u8
+// 157 / 106; 1024 x 4096 bf16 169 / 48, fp32 171 / 106; 224 rows: 4096 x 1024
+// bf16 25.5 / 10.8, fp32 25.8 / 21.3, 1024 x 4096 bf16 30.5 / 15.0, fp32 30.6
+// / 25.1. Its error against 64 bits is 0.9e-7 at K = 1024 (K-parallel kernel
+// 1.6e-7, fp32 tiles before 5.3-6.4e-7) and 2.5e-8 for a single product, as
+// fp32's. (Six products, without m l and l m, take 85 us on the first fp32
+// shape, but a sum of one product is then up to 2.5e-7 off, not 6e-8.)
 //
 // MW x NW x KW waves: MW along the tile's rows, NW along its columns, KW
 // along the contraction (each of those takes 4 / KW of a stage's four
@@ -262,17 +264,18 @@ __device__ __forceinline__ void f32_tile_body(const GemmParams& p, int splits, i
     }
   };
 
-  // The products kept (activation part, weight part): what is left out, m l,
-  // l m and l l, is below 2^-22 of a product and of either sign. h h and the
-  // others, 2^-7 of it and less, add up apart: the large sum is rounded once
-  // per 16 columns instead of once per product.
+  // The products kept (activation part, weight part), smallest first: all but
+  // l l, which is below 2^-30 of a product. h h, exact in fp32, and the
+  // others, 2^-6 of it and less, add up apart: the large sum is rounded once
+  // per 16 columns instead of once per product, and a product that makes up a
+  // sum by itself as if it were rounded from all its bits.
   floatx16 acc[2][TN][TM];
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[0][j][i] = floatx16{}, acc[1][j][i] = floatx16{};
-  constexpr int NPR = C::PB == 1 ? 3 : 6;
-  constexpr int PRA[6] = {2, 0, 1, 0, 1, 0}, PRB[6] = {0, 0, 0, 2, 1, 1};
+  constexpr int NPR = C::PB == 1 ? 3 : 8;
+  constexpr int PRA[8] = {2, 1, 2, 0, 1, 0, 1, 0}, PRB[8] = {1, 2, 0, 0, 0, 2, 1, 1};
   constexpr int PRA1[3] = {2, 0, 1};
   constexpr int NM = NPR * TM * TN, LEAD = NM / 5;
   constexpr int CG = 2;  // MFMAs (and conversion pieces) scheduled together

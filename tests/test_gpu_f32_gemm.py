@@ -3,7 +3,7 @@ remainders of their row tiles, one to many 64-column stages, every split of
 the contraction, each weight kind, and values that are not finite.
 
 The kernels write an fp32 value as the exact sum of three bf16 values and
-leave out products below 2^-22 of the whole one, so their results carry the
+leave out products below 2^-30 of the whole one, so their results carry the
 error of fp32 sums: K 2^-24 |A| |W|^T per element at most (K roundings), and
 in the 2-norm that of K / 16 roundings of random sign.
 """
@@ -78,6 +78,26 @@ def test_linear2_splits(d, f, rows, kind):
     x = rng.standard_normal((rows, f)).astype(np.float32)
     got = m.debug_linear(1, torch.from_numpy(x).cuda()).cpu().numpy()
     check(got, x.astype(np.float64), dense[1], f"linear2 {kind} {rows}x{d}x{f}")
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("which,rows", [(0, 300), (1, 40)])
+def test_sums_of_few_terms(which, rows, kind):
+    """A product that is a sum by itself is rounded as one fp32 product: half a
+    unit in the last place, 2^-24, and 2^-27 for the small parts' own sum (they
+    are 2^-6 of it, rounded 7 times) and what is left out. Two terms are
+    rounded twice more where they meet."""
+    rng = np.random.default_rng(rows)
+    m, dense = make_ff(rng, 256, 4096, kind)
+    k = 4096 if which else 256
+    for terms, bound in ((1, 2.0 ** -24 + 2.0 ** -27), (2, 3 * 2.0 ** -24 + 2.0 ** -27)):
+        x = np.zeros((rows, k), dtype=np.float32)
+        for r in range(rows):
+            x[r, rng.choice(k, terms, replace=False)] = rng.standard_normal(terms)
+        got = m.debug_linear(which, torch.from_numpy(x).cuda()).cpu().numpy().astype(np.float64)
+        x = x.astype(np.float64)
+        over = np.abs(got - x @ dense[which].T) - bound * (np.abs(x) @ np.abs(dense[which]).T)
+        assert (over <= 0).all(), f"{terms} terms: {over.max():.3g}"
 
 
 def test_rows_past_two_gib():
