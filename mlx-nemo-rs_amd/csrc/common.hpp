@@ -97,9 +97,9 @@ __device__ __forceinline__ float silu_value(float v) {
 // cut to its top 8 significant bits, m the remainder (under 2^-7 |x|) rounded
 // to bf16, and what is left, l, under 2^-15 |x|, fits bf16. This splits a
 // pair, packed as MFMA operands take them. (Parts below the smallest bf16
-// subnormal are lost: values under ~1e-33 keep fewer bits. An infinite or NaN
-// value makes m and l NaN, and so every sum it enters: the kernels recompute
-// those in plain fp32.)
+// subnormal are lost: values under 2^-110 keep fewer bits. An infinite or NaN
+// value makes m and l NaN, and so every sum it enters. The kernels recompute
+// both kinds of sums in plain fp32.)
 // (The empty asm keeps the packed word opaque: otherwise the compiler
 // converts each value once more for the subtractions.)
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {

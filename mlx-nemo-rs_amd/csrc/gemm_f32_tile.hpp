@@ -5,15 +5,16 @@
 
 enum WKind { kWF32 = 0, kWBF16 = 1, kWU8 = 2 };
 
-// A[row, :] . W[col, :] in plain fp32 (the epilogue's recomputation).
+// A[row, :] . W[col, :] in plain fp32, four chains (the epilogue's
+// recomputation).
 template <int WK>
 __device__ __forceinline__ float f32_dot(const GemmParams& p, int row, int col) {
   const float* a = reinterpret_cast<const float*>(p.A) + (int64_t)row * p.lda;
   const int64_t w0 = (int64_t)col * p.K;
-  float s = 0.f;
+  floatx4 s{};
   // (a NaN stays one: rows that hold one end at the group of 64 where it is)
 #pragma unroll 1
-  for (int k0 = 0; k0 < p.K && s == s; k0 += 64) {
+  for (int k0 = 0; k0 < p.K && s[0] == s[0] && s[1] == s[1] && s[2] == s[2] && s[3] == s[3]; k0 += 64) {
 #pragma unroll 4
     for (int k = k0; k < k0 + 64; k += 4) {
       const floatx4 av = *reinterpret_cast<const floatx4*>(a + k);
@@ -30,20 +31,26 @@ __device__ __forceinline__ float f32_dot(const GemmParams& p, int row, int col) 
         for (int e = 0; e < 4; ++e) w[e] = __builtin_fmaf(sb[0], (float)((c >> (8 * e)) & 0xFFu), sb[1]);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s = __builtin_fmaf(av[e], w[e], s);
+      for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(av[e], w[e], s[e]);
     }
   }
-  return s;
+  return (s[0] + s[1]) + (s[2] + s[3]);
 }
+
+// Values under 2^-110 have parts below the smallest bf16, 2^-133, which are
+// lost: up to 2^-134 of each. A sum of at least this, of up to 2^14 products
+// with weights up to 2^8, is off by no more than 2^-26 of it.
+constexpr float kF32Small = 0x1p-86f;
 
 // Columns [col, col + 4) of a row: the sums `v`, then the epilogue in the
 // reference's order (bias, SiLU, scaled residual) and the store.
 template <int WK>
 __device__ __forceinline__ void f32_store(const GemmParams& p, int row, int col, floatx4 v) {
-  if (__any(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3])) {
+  auto whole = [](float x) { return __builtin_fabsf(x) >= kF32Small; };  // (not so for NaN)
+  if (__any(!whole(v[0]) || !whole(v[1]) || !whole(v[2]) || !whole(v[3]))) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (v[e] != v[e]) v[e] = f32_dot<WK>(p, row, col + e);
+      if (!whole(v[e]) && v[e] != 0.f) v[e] = f32_dot<WK>(p, row, col + e);
   }
   if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + col);
   if (p.act == kActSilu) {

@@ -147,6 +147,30 @@ def test_scaled_inputs(scale):
     check(got, x.astype(np.float64), dense[0], f"scale {scale}")
 
 
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("which,rows", [(0, 160), (1, 40)])
+def test_tiny_values(which, rows, kind):
+    """Rows whose values are too small for three bf16 parts (under 2^-110),
+    beside ordinary and zero rows, and an ordinary row of some tiny values.
+    Products below the smallest normal number, 2^-126, lose up to 2^-150."""
+    rng = np.random.default_rng(11)
+    m, dense = make_ff(rng, 256, 4096, kind)
+    k = 4096 if which else 256
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    for r, scale in ((1, -112), (2, -116), (5, -119), (6, -122)):
+        x[r] *= np.float32(2.0 ** scale)
+    x[9, ::2] *= np.float32(2.0 ** -118)
+    x[12] = 0
+    got = m.debug_linear(which, torch.from_numpy(x).cuda()).cpu().numpy().astype(np.float64)
+    x = x.astype(np.float64)
+    ref, mag = x @ dense[which].T, np.abs(x) @ np.abs(dense[which]).T
+    assert (np.abs(got - ref) <= k * (2.0 ** -24 * mag + 2.0 ** -149)).all()
+    for r in (1, 2, 5):
+        rel = np.linalg.norm(got[r] - ref[r]) / np.linalg.norm(ref[r])
+        assert rel <= 2.0 ** -20, f"row {r}: {rel:.2e}"
+    assert not got[12].any()
+
+
 # one utterance's Q/K/V and position projections in one launch, with 1 to 3
 # row tiles each; the result is that of the two apart
 @pytest.mark.parametrize("quant", [False, True])
