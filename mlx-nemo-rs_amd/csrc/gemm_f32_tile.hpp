@@ -5,53 +5,111 @@
 
 enum WKind { kWF32 = 0, kWBF16 = 1, kWU8 = 2 };
 
-// A[row, :] . W[col, :] in plain fp32, four chains (the epilogue's
-// recomputation).
+// A[row, :] . W[col + c, :], c = 0..3, in plain fp32, four chains each (the
+// epilogue's recomputation).
 template <int WK>
-__device__ __forceinline__ float f32_dot(const GemmParams& p, int row, int col) {
+__device__ __forceinline__ floatx4 f32_dot4(const GemmParams& p, int row, int col) {
   const float* a = reinterpret_cast<const float*>(p.A) + (int64_t)row * p.lda;
   const int64_t w0 = (int64_t)col * p.K;
-  floatx4 s{};
-  // (a NaN stays one: rows that hold one end at the group of 64 where it is)
+  floatx4 s[4] = {};
 #pragma unroll 1
-  for (int k0 = 0; k0 < p.K && s[0] == s[0] && s[1] == s[1] && s[2] == s[2] && s[3] == s[3]; k0 += 64) {
+  for (int k0 = 0; k0 < p.K; k0 += 64) {
+    floatx2 sb[4];
+    if constexpr (WK == kWU8) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        sb[c] = *reinterpret_cast<const floatx2*>(p.sb + 2 * ((int64_t)(col + c) * (p.K / 64) + k0 / 64));
+    }
 #pragma unroll 4
     for (int k = k0; k < k0 + 64; k += 4) {
       const floatx4 av = *reinterpret_cast<const floatx4*>(a + k);
-      floatx4 w;
-      if constexpr (WK == kWF32) {
-        w = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(p.W) + w0 + k);
-      } else if constexpr (WK == kWBF16) {
-        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16*>(p.W16) + w0 + k);
-        w = floatx4{(float)wv[0], (float)wv[1], (float)wv[2], (float)wv[3]};
-      } else {
-        const float* sb = p.sb + 2 * ((int64_t)col * (p.K / 64) + k0 / 64);
-        const uint32_t c = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(p.W) + w0 + k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = __builtin_fmaf(sb[0], (float)((c >> (8 * e)) & 0xFFu), sb[1]);
+      for (int c = 0; c < 4; ++c) {
+        const int64_t at = w0 + (int64_t)c * p.K + k;
+        floatx4 w;
+        if constexpr (WK == kWF32) {
+          w = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(p.W) + at);
+        } else if constexpr (WK == kWBF16) {
+          const bf16x4 wv = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16*>(p.W16) + at);
+          w = floatx4{(float)wv[0], (float)wv[1], (float)wv[2], (float)wv[3]};
+        } else {
+          const uint32_t q = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(p.W) + at);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = __builtin_fmaf(sb[c].x, (float)((q >> (8 * e)) & 0xFFu), sb[c].y);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[c][e] = __builtin_fmaf(av[e], w[e], s[c][e]);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(av[e], w[e], s[e]);
     }
   }
-  return (s[0] + s[1]) + (s[2] + s[3]);
+  floatx4 r;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) r[c] = (s[c][0] + s[c][1]) + (s[c][2] + s[c][3]);
+  return r;
 }
 
 // Values under 2^-110 have parts below the smallest bf16, 2^-133, which are
 // lost: up to 2^-134 of each. A sum of at least this, of up to 2^14 products
-// with weights up to 2^8, is off by no more than 2^-26 of it.
+// with weights up to 2^8, is off by no more than 2^-26 of it. (A matrix of
+// nothing else takes 10 to 15 times a launch, each weight read by every lane.)
 constexpr float kF32Small = 0x1p-86f;
 
-// Columns [col, col + 4) of a row: the sums `v`, then the epilogue in the
-// reference's order (bias, SiLU, scaled residual) and the store.
+// A lane's sums that are not numbers of full precision, run by whole waves.
+// Sums that are not finite come from leading parts alone (f32_sum), which
+// carry an infinite value as it is, so what is left to know is the row's: with
+// a NaN in it (whose leading part may be an infinity) every sum is NaN, with
+// an infinity the sum stands, without either (an overflow, a weight that is
+// not finite) it is recomputed, as small ones are. The wave reads a row once
+// for all its lanes: recomputing each sum of rows with an infinity took up to
+// 18 times a launch.
 template <int WK>
-__device__ __forceinline__ void f32_store(const GemmParams& p, int row, int col, floatx4 v) {
-  auto whole = [](float x) { return __builtin_fabsf(x) >= kF32Small; };  // (not so for NaN)
-  if (__any(!whole(v[0]) || !whole(v[1]) || !whole(v[2]) || !whole(v[3]))) {
+__device__ __forceinline__ void f32_mend(const GemmParams& p, bool ok, int row, int col, floatx4& v) {
+  bool odd = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (!whole(v[e]) && v[e] != 0.f) v[e] = f32_dot<WK>(p, row, col + e);
+  for (int e = 0; e < 4; ++e) odd = odd || (ok && !(__builtin_fabsf(v[e]) < INFINITY));
+  bool has_nan = false, has_inf = false;
+  for (uint64_t left = __ballot(odd); left;) {
+    const int r = __builtin_amdgcn_readlane(row, __builtin_ctzll(left));
+    const float* a = reinterpret_cast<const float*>(p.A) + (int64_t)r * p.lda;
+    bool n = false, i = false;
+    for (int k = 4 * (int)(threadIdx.x & 63); k < p.K; k += 256) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(a + k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) n = n || x[e] != x[e], i = i || __builtin_fabsf(x[e]) == INFINITY;
+    }
+    n = __any(n), i = __any(i);
+    if (row == r) has_nan = n, has_inf = i;
+    left &= ~__ballot(row == r);
   }
+  bool again[4], any = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool finite = __builtin_fabsf(v[e]) < INFINITY;
+    again[e] = ok && (finite ? v[e] != 0.f && __builtin_fabsf(v[e]) < kF32Small : !has_nan && !has_inf);
+    any = any || again[e];
+    if (!finite && has_nan) v[e] = NAN;
+  }
+  if (any) {
+    const floatx4 d = f32_dot4<WK>(p, row, col);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = again[e] ? d[e] : v[e];
+  }
+}
+
+// The sum of a wave's accumulators: an infinite or NaN value's lower parts are
+// NaN, and its leading products alone say what its sums are.
+__device__ __forceinline__ float f32_sum(float lead, float rest) {
+  return __builtin_fabsf(lead) < INFINITY ? lead + rest : lead;
+}
+
+// Columns [col, col + 4) of a row: the sums `v`, then the epilogue in the
+// reference's order (bias, SiLU, scaled residual) and the store. Whole waves,
+// `ok` where there is such a row.
+template <int WK>
+__device__ __forceinline__ void f32_store(const GemmParams& p, bool ok, int row, int col, floatx4 v) {
+  auto whole = [](float x) { return __builtin_fabsf(x) >= kF32Small && __builtin_fabsf(x) < INFINITY; };
+  if (__any(ok && !(whole(v[0]) && whole(v[1]) && whole(v[2]) && whole(v[3])))) f32_mend<WK>(p, ok, row, col, v);
+  if (!ok) return;
   if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + col);
   if (p.act == kActSilu) {
 #pragma unroll
@@ -373,9 +431,10 @@ __device__ __forceinline__ void f32_tile_body(const GemmParams& p, int splits, i
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *reinterpret_cast<floatx4*>(st + (i - ep * (TM / C::EPP)) * 32 * C::PITCH + (32 * j + 8 * q) * 4) =
-              floatx4{acc[0][j][i][4 * q] + acc[1][j][i][4 * q], acc[0][j][i][4 * q + 1] + acc[1][j][i][4 * q + 1],
-                      acc[0][j][i][4 * q + 2] + acc[1][j][i][4 * q + 2],
-                      acc[0][j][i][4 * q + 3] + acc[1][j][i][4 * q + 3]};
+              floatx4{f32_sum(acc[0][j][i][4 * q], acc[1][j][i][4 * q]),
+                      f32_sum(acc[0][j][i][4 * q + 1], acc[1][j][i][4 * q + 1]),
+                      f32_sum(acc[0][j][i][4 * q + 2], acc[1][j][i][4 * q + 2]),
+                      f32_sum(acc[0][j][i][4 * q + 3], acc[1][j][i][4 * q + 3])};
     __syncthreads();
     constexpr int CR = BN / 4, NCH = MW * C::EROWS * CR;  // runs per row, runs per pass
     static_assert(NCH % C::NT == 0, "runs per thread");
@@ -385,15 +444,14 @@ __device__ __forceinline__ void f32_tile_body(const GemmParams& p, int splits, i
       const int bm = er / C::EROWS, r = er % C::EROWS, bn = cc / C::WN;
       const int row = m0 + bm * C::WM + ep * C::EROWS + r, col = n0 + cc;
       const char* src = smem + (bm * NW + bn) * KW * C::EREG + r * C::PITCH + (cc - bn * C::WN) * 4;
-      if (row >= m_end) continue;
       floatx4 v = *reinterpret_cast<const floatx4*>(src);
 #pragma unroll
       for (int k = 1; k < KW; ++k) v += *reinterpret_cast<const floatx4*>(src + k * C::EREG);
       if (splits > 1) {
-        *reinterpret_cast<floatx4*>(p.partial + ((int64_t)z * p.M + row) * p.N + col) = v;
+        if (row < m_end) *reinterpret_cast<floatx4*>(p.partial + ((int64_t)z * p.M + row) * p.N + col) = v;
         continue;
       }
-      f32_store<WK>(p, row, col, v);
+      f32_store<WK>(p, row < m_end, row, col, v);
     }
   }
 }
@@ -410,9 +468,12 @@ template <int WK>
 __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmParams p, int splits) {
   const int64_t total = (int64_t)p.M * p.N;
   const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (e >= total) return;
-  floatx4 v = *reinterpret_cast<const floatx4*>(p.partial + e);
+  const bool ok = e < total;
+  floatx4 v{};
+  if (ok) {
+    v = *reinterpret_cast<const floatx4*>(p.partial + e);
 #pragma unroll 4
-  for (int z = 1; z < splits; ++z) v += *reinterpret_cast<const floatx4*>(p.partial + z * total + e);
-  f32_store<WK>(p, (int)(e / p.N), (int)(e % p.N), v);
+    for (int z = 1; z < splits; ++z) v += *reinterpret_cast<const floatx4*>(p.partial + z * total + e);
+  }
+  f32_store<WK>(p, ok, (int)(e / p.N), (int)(e % p.N), v);
 }

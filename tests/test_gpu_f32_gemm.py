@@ -137,6 +137,66 @@ def test_values_that_are_not_finite(which, rows, kind):
     check(got[rest], x[rest].astype(np.float64), dense[which], f"rows beside them, {kind}")
 
 
+@pytest.mark.parametrize("kind", ["f32", "bf16", "u8"])
+@pytest.mark.parametrize("which,rows", [(0, 321), (1, 45)])
+def test_rows_of_infinities_and_nans(which, rows, kind):
+    """Whole rows and columns that are not finite, a NaN whose leading bits are
+    an infinity's, infinities that meet weights of zero, overflows of finite
+    rows, and a weight that is not finite: what plain fp32 sums give."""
+    rng = np.random.default_rng(5 + rows)
+    m, dense = make_ff(rng, 128, 2048, kind)
+    if kind != "u8":
+        w = {"f.linear%d.weight" % (i + 1): d.astype(np.float32) for i, d in enumerate(dense)}
+        w["f.linear%d.weight" % (which + 1)][3, :32] = 0
+        w["f.linear%d.weight" % (which + 1)][5, 7] = -np.inf
+        m.load_weights(w, "f")
+        dense = [w["f.linear1.weight"].astype(np.float64), w["f.linear2.weight"].astype(np.float64)]
+    k = 2048 if which else 128
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[rows - 1, 40] = x[4, 0] = np.inf
+    x[5], x[6], x[7], x[8, ::2] = np.inf, -np.inf, np.nan, -np.inf
+    x[9, 100] = np.uint32(0x7F800001).view(np.float32)  # (a NaN with no bit in its leading half)
+    x[10] = 0
+    x[11, 2] = np.float32(3e38)
+    got = m.debug_linear(which, torch.from_numpy(x).cuda()).cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = x.astype(np.float64) @ dense[which].T
+        r32 = ref.astype(np.float32)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(r32))
+    np.testing.assert_array_equal(np.where(np.isinf(r32), r32, 0), np.where(np.isinf(got), got, 0))
+    rest = np.setdiff1d(np.arange(rows), [4, 5, 6, 7, 8, 9, 11, rows - 1])
+    cols = np.isfinite(dense[which]).all(axis=1)
+    check(got[rest][:, cols], x[rest].astype(np.float64), dense[which][cols], f"rows beside them, {kind}")
+
+
+@pytest.mark.parametrize("kind", ["f32", "u8"])
+def test_time_of_rows_that_are_not_finite(kind):
+    """Rows with NaNs or infinities cost a reading of the row (1.3 times a
+    launch where every row has one), not a recomputation of its sums (11 to 18
+    times)."""
+    rng = np.random.default_rng(2)
+    m, _ = make_ff(rng, 1024, 4096, kind)
+    x = torch.randn((1500, 1024), generator=torch.Generator("cuda").manual_seed(2), device="cuda")
+
+    def best(x):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                m.forward(x)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    plain = best(x)
+    for value in (float("nan"), float("inf")):
+        y = x.clone()
+        y[:, 3] = value
+        assert best(y) < 4 * plain, value
+
+
 @pytest.mark.parametrize("scale", [1e-20, 1e-3, 1e4, 1e18])
 def test_scaled_inputs(scale):
     """The parts keep 24 bits over the fp32 range, not around 1 alone."""
