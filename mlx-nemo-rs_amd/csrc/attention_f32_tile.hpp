@@ -7,9 +7,12 @@
 // workgroup each. The fp32 MFMA bounded it (157 TFLOP/s; the kernel reached a
 // quarter of that), so K, V, the position rows, the queries and the
 // probabilities go through the bf16 MFMAs as three exact bf16 parts each
-// (split_pair), six products per pair of values: what is left out is below
-// 2^-22 of a product. In the scores the product of the leading parts and the
-// others add up apart, so a large sum is rounded once per 32 terms.
+// (split_pair), eight products per pair of values: what is left out is below
+// 2^-30 of a product. In the scores the product of the leading parts, exact in
+// fp32, and the others add up apart, so a large sum is rounded once per 32
+// terms, and one that a product makes up as the product of all its bits. (Six
+// products leave out up to 2^-22: a score of one large product was then up to
+// 2.5e-7 of it off, 6.0e-8 so.)
 //
 // A workgroup of 4 waves owns 64 queries of one (batch, head), 16 a wave, and
 // walks the keys in tiles of 32. Rows are split once per workgroup, on their
@@ -212,9 +215,9 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
 #pragma unroll
     for (int t = 0; t < 3; ++t) a[t] = *reinterpret_cast<const bf16x8*>(at + t * part_bytes);
   };
-  // the six products of two values in parts, smallest first (part of the
+  // the eight products of two values in parts, smallest first (part of the
   // row, part of the query or probability)
-  constexpr int PRA[6] = {2, 0, 1, 1, 0, 0}, PRB[6] = {0, 2, 1, 0, 1, 0};
+  constexpr int NX = 8, PRA[NX] = {2, 1, 2, 0, 1, 1, 0, 0}, PRB[NX] = {1, 2, 0, 2, 1, 0, 1, 0};
 
   floatx4 o[ND];
 #pragma unroll
@@ -268,20 +271,20 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
         parts(smem + C::P_OFF + (brow[n] + ql) * C::RB + swz(ql, 4 * kf + g), C::PPART, pa[n]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int x = 0; x < 6; ++x)
+      for (int x = 0; x < NX; ++x)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          floatx4& d = x < 5 ? sl[u] : sh[u];
+          floatx4& d = x < NX - 1 ? sl[u] : sh[u];
           d = mma16(ka[u][PRA[x]], __builtin_bit_cast(bf16x8, qu[kf][PRB[x]]), d);
         }
       __builtin_amdgcn_sched_barrier(0);
       if (kf + 1 < NKF) read_k(kf + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int x = 0; x < 6; ++x)
+      for (int x = 0; x < NX; ++x)
 #pragma unroll
         for (int n = 0; n < 3; ++n) {
-          floatx4& d = x < 5 ? bl3[n] : bh[n];
+          floatx4& d = x < NX - 1 ? bl3[n] : bh[n];
           d = mma16(pa[n][PRA[x]], __builtin_bit_cast(bf16x8, qv[kf][PRB[x]]), d);
         }
       __builtin_amdgcn_sched_barrier(0);
@@ -335,19 +338,19 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
       for (int x = 0; x < 2; ++x)
         parts(smem + C::V_OFF + (32 * d2 + 16 * x + ql) * C::VP + 16 * g, C::VPART, va[d2 & 1][x]);
     };
-    constexpr int NMM = 6 * ND;
+    constexpr int NMM = NX * ND;
     read_v(0);
 #pragma unroll
     for (int d2 = 0; d2 < ND / 2; ++d2) {
       if (d2 + 1 < ND / 2) read_v(d2 + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int x = 0; x < 6; ++x) {
+      for (int x = 0; x < NX; ++x) {
 #pragma unroll
         for (int y = 0; y < 2; ++y)
           o[2 * d2 + y] = mma16(va[d2 & 1][y][PRA[x]], __builtin_bit_cast(bf16x8, pb[PRB[x]]), o[2 * d2 + y]);
         constexpr int LEAD = ND;  // (the rows' loads get a first part of the products to land)
-        const int mm = 12 * d2 + 2 * x;
+        const int mm = 2 * NX * d2 + 2 * x;
 #pragma unroll
         for (int c = 0; c < NPIECE; ++c)
           if (LEAD + c * (NMM - LEAD) / NPIECE / 2 * 2 == mm) split_piece(c);

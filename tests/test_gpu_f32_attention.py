@@ -3,7 +3,7 @@ query blocks and key tiles that end inside a tile, one tile to many turns of
 the position ring, contexts that start inside a block, items of different
 lengths, and values that are not finite.
 
-The products left out are below 2^-22 of the whole one, and the sums are fp32:
+The products left out are below 2^-30 of the whole one, and the sums are fp32:
 the error in the 2-norm is that of the projections and the attention at a few
 roundings of random sign each, 2^-19 at most (measured 2^-21).
 """
@@ -60,6 +60,54 @@ def test_forward_against_oracle(d, h, B, T, ctx):
         rows = np.isfinite(ref).all(axis=-1)
         err = np.linalg.norm(got[b:b + 1][rows] - ref[rows]) / np.linalg.norm(ref[rows])
         assert rows.any() and err < 2.0 ** -19, (b, err)
+
+
+@pytest.mark.parametrize("d,h", [(512, 8), (256, 2)])
+def test_scores_of_one_product(d, h):
+    """Scores that one product makes up (around 250 and 180), two keys a query:
+    the output is one key's probability, and its logit the difference of the
+    two scores. Each is rounded as an fp32 product (2^-24 and, for the parts'
+    own sum, 2^-27) and once more when it is scaled; the probability's
+    roundings weigh up to 10 times as much in the logit, under 100 2^-24 in
+    all. The values have large second and third parts, of which the own key's
+    and the other's third differ in sign; roundings are spread evenly, so half
+    of the errors are below half their bound."""
+    B, T, dk = 128 // h, 64, d // h
+    rng = np.random.default_rng(d)
+    w = {"l.%s.weight" % n: np.zeros((d, d), dtype=np.float32)
+         for n in ("linear_q", "linear_k", "linear_v", "linear_out", "linear_pos")}
+    for i in range(h):
+        for c, n in enumerate(("linear_q", "linear_k", "linear_v")):
+            w["l.%s.weight" % n][i * dk, 3 * i + c] = 1
+        w["l.linear_out.weight"][i, i * dk] = 1
+    w["l.pos_bias_u"] = w["l.pos_bias_v"] = np.zeros((h, dk), dtype=np.float32)
+    layer = M.RelPositionMultiHeadAttention(d, h, False)
+    layer.load_weights(w, "l")
+    layer.set_dtype(O.F32)
+    x = np.zeros((B, T, d), dtype=np.float32)
+    ulp = 2.0 ** -23
+    steps = lambda: rng.integers(1, 40, (B, T, h)) * ulp  # noqa: E731
+    q = (16 * (1 + 255 * 2.0 ** -15 + 2.0 ** -16 - steps())).astype(np.float32)
+    k = (128 * (1 + 255 * 2.0 ** -15 + 2.0 ** -16 - steps())).astype(np.float32)
+    k[:, 1::2] = (128 * (1 + 2.0 ** -15 - 2.0 ** -16 + steps())[:, 1::2]).astype(np.float32)
+    even = (np.arange(T) % 2 == 0).astype(np.float32)
+    for i in range(h):
+        x[:, :, 3 * i], x[:, :, 3 * i + 1], x[:, :, 3 * i + 2] = q[..., i], k[..., i], even
+    pos = O.RelPositionalEncoding(d, 5000, True).get_encoding(T)
+    before = M.debug_attention_forms()["generic"]
+    got = layer.forward(torch.from_numpy(x).cuda(), torch.from_numpy(pos).float().cuda().contiguous(),
+                        M.AttentionContext.new((1, 0), "regular"), None).cpu().numpy().astype(np.float64)
+    assert M.debug_attention_forms()["generic"] == before + 1
+    q, k = q.astype(np.float64)[:, 1:], k.astype(np.float64)
+    s = np.stack([q * k[:, :-1], q * k[:, 1:]]) / np.sqrt(dk)  # of the key before, of its own
+    p = got[:, 1:, :h]
+    first = (even[:-1] == 1)[None, :, None]
+    diff = np.where(first, s[0] - s[1], s[1] - s[0])
+    use = (p > 0.1) & (p < 0.9)
+    err = np.abs(np.log(p[use] / (1 - p[use])) - diff[use])
+    bound = (2 + 2.0 ** -3) * 2.0 ** -24 * s.sum(axis=0)[use] + 100 * 2.0 ** -24
+    assert use.sum() > 1000 and (err <= bound).all(), f"{np.max(err / bound):.3g} of the bound"
+    assert np.median(err / bound) <= 0.5, f"half are above {np.median(err / bound):.3g} of the bound"
 
 
 def test_values_that_are_not_finite():
