@@ -44,43 +44,71 @@ struct F32Attn {
   static_assert(KC >= 1 && (VK == 2 || VK == 4) && LDS <= 160 * 1024, "tile split");
 };
 
-// One query in plain fp32, lane l on columns l and l + 64 (for the queries
-// whose sums met a value that the parts cannot carry).
+// One query in plain fp32 by one wave (for the queries whose sums met a value
+// that the parts cannot carry): 64 keys at a time, a key per lane for the
+// scores, columns l and l + 64 per lane for the output. A NaN in the query or
+// among the visible scores makes the output NaN and ends it.
 template <int DK>
 __device__ __forceinline__ void attn_f32_plain(const AttnParams& p, int bl, int h, int i, float sc_qk, float sc_bd) {
   constexpr int N = DK / 64;
-  const int lane = threadIdx.x & 63, b = p.b0 + bl, c = h * DK + lane;
-  const float* q = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_bs + (int64_t)i * p.q_rs + c;
-  const float* kb = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.kv_bs + c;
-  const float* vb = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.kv_bs + c;
-  const float* pb = reinterpret_cast<const float*>(p.p) + c;
-  float qu[N], qv[N], o[N], m = -INFINITY, l = 0.f;
+  const int lane = threadIdx.x & 63, b = p.b0 + bl;
+  const float* q = reinterpret_cast<const float*>(p.q) + (int64_t)b * p.q_bs + (int64_t)i * p.q_rs + h * DK;
+  const float* kb = reinterpret_cast<const float*>(p.k) + (int64_t)b * p.kv_bs + h * DK;
+  const float* vb = reinterpret_cast<const float*>(p.v) + (int64_t)b * p.kv_bs + h * DK + lane;
+  const float* pb = reinterpret_cast<const float*>(p.p) + h * DK;
+  float* orow = reinterpret_cast<float*>(p.o) + (int64_t)b * p.o_bs + (int64_t)i * p.o_rs + h * DK + lane;
+  float o[N], m = -INFINITY, l = 0.f;
+  bool nan = false;
 #pragma unroll
-  for (int n = 0; n < N; ++n) qu[n] = q[64 * n] + p.bias_u[c + 64 * n], qv[n] = q[64 * n] + p.bias_v[c + 64 * n], o[n] = 0.f;
+  for (int n = 0; n < N; ++n) {
+    const float x = q[lane + 64 * n];
+    o[n] = 0.f;
+    nan = nan || x != x;
+  }
   const int2 iv = query_interval(p, bl, i);
+  nan = __any(nan) && iv.x < iv.y;
 #pragma unroll 1
-  for (int j = iv.x; j < iv.y; ++j) {
-    const int64_t row = (int64_t)key_row(p, j) * p.kv_rs;
-    const int tp = p.center - p.qoff - i + j;
+  for (int j0 = iv.x; j0 < iv.y && !nan; j0 += 64) {
+    const int j = min(j0 + lane, iv.y - 1), tp = p.center - p.qoff - i + j;
     const bool ok = tp >= 0 && tp < p.p_rows;
-    float s = 0.f, t = 0.f;
+    const int64_t row = (int64_t)key_row(p, j) * p.kv_rs;
+    const float* prow = pb + (int64_t)(ok ? tp : 0) * p.p_rs;
+    floatx4 s{}, t{};
+#pragma unroll 4
+    for (int d = 0; d < DK; d += 4) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(q + d);
+      const floatx4 k = *reinterpret_cast<const floatx4*>(kb + row + d);
+      const floatx4 r = *reinterpret_cast<const floatx4*>(prow + d);
 #pragma unroll
-    for (int n = 0; n < N; ++n) {
-      s += qu[n] * kb[row + 64 * n];
-      t += qv[n] * (ok ? pb[(int64_t)tp * p.p_rs + 64 * n] : 0.f);
+      for (int e = 0; e < 4; ++e) {
+        s[e] = __builtin_fmaf(x[e] + p.bias_u[h * DK + d + e], k[e], s[e]);
+        t[e] = __builtin_fmaf(x[e] + p.bias_v[h * DK + d + e], ok ? r[e] : 0.f, t[e]);
+      }
     }
-    for (int x = 32; x > 0; x >>= 1) s += __shfl_xor(s, x, 64), t += __shfl_xor(t, x, 64);
-    const float v = s * sc_qk + t * sc_bd, mn = fmaxf(m, v), mu = mn == -INFINITY ? 0.f : mn;
-    const float alpha = __builtin_amdgcn_exp2f(m - mu), e = __builtin_amdgcn_exp2f(v - mu);
+    float v = ((s[0] + s[1]) + (s[2] + s[3])) * sc_qk + ((t[0] + t[1]) + (t[2] + t[3])) * sc_bd;
+    if (j0 + lane >= iv.y) v = -INFINITY;
+    float mn = fmaxf(m, v);
+    for (int x = 32; x > 0; x >>= 1) mn = fmaxf(mn, __shfl_xor(mn, x, 64));
+    const float mu = mn == -INFINITY ? 0.f : mn, alpha = __builtin_amdgcn_exp2f(m - mu);
+    const float e = __builtin_amdgcn_exp2f(v - mu);
     m = mn;
     l = l * alpha + e;
+    nan = __any(l != l);
+    if (nan) break;
 #pragma unroll
-    for (int n = 0; n < N; ++n) o[n] = o[n] * alpha + e * vb[row + 64 * n];
+    for (int n = 0; n < N; ++n) o[n] *= alpha;
+    const int keys = min(64, iv.y - j0);
+    for (int x = 0; x < keys; ++x) {
+      const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), x));
+      const float* vr = vb + (int64_t)key_row(p, j0 + x) * p.kv_rs;
+#pragma unroll
+      for (int n = 0; n < N; ++n) o[n] = __builtin_fmaf(w, vr[64 * n], o[n]);
+    }
   }
+  for (int x = 32; x > 0; x >>= 1) l += __shfl_xor(l, x, 64);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  float* orow = reinterpret_cast<float*>(p.o) + (int64_t)b * p.o_bs + (int64_t)i * p.o_rs + c;
 #pragma unroll
-  for (int n = 0; n < N; ++n) orow[64 * n] = o[n] * inv;
+  for (int n = 0; n < N; ++n) orow[64 * n] = nan ? NAN : o[n] * inv;
 }
 
 template <int DK>
@@ -128,8 +156,9 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
   const int jfirst = jbeg / NK * NK, ntile = jend > jfirst ? (jend - jfirst + NK - 1) / NK : 0;
   const int pmin = p.center - p.qoff - (i0 + QB - 1) + jfirst;  // position row of ring block 0, row 0
 
-  // Loads are unconditional: rows past the last key or outside the table
-  // read row 0 and become zeros. Chunk x of this thread: row and 8 columns.
+  // Loads are unconditional: rows of keys that no query of the block sees
+  // (padding may hold anything) or outside the table read row 0 and become
+  // zeros. Chunk x of this thread: row and 8 columns.
   floatx4 kr[C::KC][2], pr[C::KC][2], vr[C::VK];
   const int vkq = tid % (NK / C::VK), vd = tid / (NK / C::VK) * 4;  // V: keys VK vkq + [0, VK), columns vd + [0, 4)
   auto crow = [&](int x) { return (tid + x * C::NT) / (DK / 8); };
@@ -138,7 +167,7 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
 #pragma unroll
     for (int x = 0; x < C::KC; ++x) {
       const int j = j0 + crow(x);
-      const bool ok = j < p.L;
+      const bool ok = j >= jbeg && j < jend;
       const float* src = kbase + (int64_t)(ok ? key_row(p, j) : 0) * p.kv_rs + ccol(x);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
@@ -149,7 +178,7 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
 #pragma unroll
     for (int x = 0; x < C::VK; ++x) {
       const int j = j0 + C::VK * vkq + x;
-      const bool ok = j < p.L;
+      const bool ok = j >= jbeg && j < jend;
       const floatx4 v = *reinterpret_cast<const floatx4*>(vbase + (int64_t)(ok ? key_row(p, j) : 0) * p.kv_rs + vd);
       vr[x] = ok ? v : floatx4{0.f, 0.f, 0.f, 0.f};
     }
@@ -370,11 +399,13 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
     odd = odd || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
     if (qi < p.T) *reinterpret_cast<floatx4*>(orow + 16 * d + 4 * g) = v;
   }
-  if (__any(odd && qi < p.T)) {
-    // an infinite or NaN value, or an overflow between parts: these 16
-    // queries again in plain fp32
+  // queries that met an infinite or NaN value, or an overflow between parts,
+  // again in plain fp32 (a layer of 4 x 375 frames, 8 heads of 128: 199 us, 230
+  // with three items half padding of NaNs, 333 with a frame of infinities that
+  // every query of an item sees)
+  uint64_t redo = __ballot(odd && qi < p.T);
+  redo |= redo >> 32, redo |= redo >> 16;
 #pragma unroll 1
-    for (int e = 0; e < 16; ++e)
-      if (i0 + 16 * w + e < p.T) attn_f32_plain<DK>(p, bl, h, i0 + 16 * w + e, sc_qk, sc_bd);
-  }
+  for (uint32_t left = (uint32_t)redo & 0xFFFFu; left; left &= left - 1)
+    attn_f32_plain<DK>(p, bl, h, i0 + 16 * w + __builtin_ctz(left), sc_qk, sc_bd);
 }

@@ -124,3 +124,59 @@ def test_values_that_are_not_finite():
     assert np.array_equal(got[keep], clean[keep])
     err = np.linalg.norm(got[3, :70] - clean[3, :70]) / np.linalg.norm(clean[3, :70])
     assert err < 2.0 ** -19, err
+
+
+@pytest.mark.parametrize("d,h,B,T,ctx", [(512, 8, 16, 100, None), (1024, 8, 4, 225, None),
+                                         (512, 8, 4, 225, ((40, 7), "regular")), (256, 2, 32, 130, ((20, 20), "regular"))])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_frames_that_are_not_finite(d, h, B, T, ctx, value):
+    """Frames of NaNs or infinities at both ends, in the middle and in the
+    padding: a query that sees one, or is one and sees any, is NaN, as its
+    scores are, and every other query is what it is without them."""
+    rng, layer, p, pos = make(d, h, T, d + B)
+    x = rng.standard_normal((B, T, d)).astype(np.float32)
+    lengths = [T, T - 60, T, T - 33] + [T - 5] * (B - 4)
+    context = M.AttentionContext.new(*ctx) if ctx else None
+    clean = forward(layer, x, pos, context, lengths, T)
+    x[0, T - 1, 3], x[1, T - 60:], x[2, 70], x[3, T - 20] = value, value, value, value
+    got = forward(layer, x, pos, context, lengths, T)
+    for b in range(min(B, 5)):
+        i, j = np.arange(T)[:, None], np.arange(T)[None]
+        seen = (j < lengths[b]) & ((j >= i - ctx[0][0]) & (j <= i + ctx[0][1]) if ctx else True)
+        bad = ~np.isfinite(x[b]).all(axis=1)
+        hit = (seen & bad[None]).any(axis=1) | (bad & seen.any(axis=1))
+        assert np.isnan(got[b][hit]).all(), b
+        ok = seen.any(axis=1) & ~hit
+        if ok.any():
+            err = np.linalg.norm(got[b][ok] - clean[b][ok]) / np.linalg.norm(clean[b][ok])
+            assert err < 2.0 ** -19, (b, err)
+
+
+def test_time_of_frames_that_are_not_finite():
+    """A launch with NaNs in the padding, or an infinity that every query of an
+    item sees, takes no more than 4 times an ordinary one (measured 1.2 and
+    1.7; 9 to 15 times where every such query walked its keys one by one)."""
+    B, T = 4, 375
+    rng, layer, p, pos = make(1024, 8, T, 3)
+    x = torch.randn((B, T, 1024), generator=torch.Generator("cuda").manual_seed(3), device="cuda")
+    pos = torch.from_numpy(pos).float().cuda().contiguous()
+    keys = M.key_padding_mask([T] + [T // 2] * (B - 1), T)
+
+    def best(x):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                layer.forward(x, pos, None, keys)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    plain = best(x)
+    padded, infinite = x.clone(), x.clone()
+    padded[1:, T // 2:] = float("nan")
+    infinite[1, 3] = float("inf")
+    assert best(padded) < 4 * plain
+    assert best(infinite) < 4 * plain
