@@ -44,6 +44,11 @@ struct F32Attn {
   static_assert(KC >= 1 && (VK == 2 || VK == 4) && LDS <= 160 * 1024, "tile split");
 };
 
+// V's values under 2^-110 have parts below the smallest bf16, 2^-133, which are
+// lost: up to 2^-134 of each, and so of their mean, 2^-48 of this. (In the
+// scores such values do not show.)
+constexpr float kF32AttnSmall = 0x1p-86f;
+
 // One query in plain fp32 by one wave (for the queries whose sums met a value
 // that the parts cannot carry): 64 keys at a time, a key per lane for the
 // scores, columns l and l + 64 per lane for the output. A NaN in the query or
@@ -396,11 +401,15 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
 #pragma unroll
   for (int d = 0; d < ND; ++d) {
     const floatx4 v = o[d] * inv;
-    odd = odd || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = __builtin_fabsf(v[e]);
+      odd = odd || !(a >= kF32AttnSmall || a == 0.f);
+    }
     if (qi < p.T) *reinterpret_cast<floatx4*>(orow + 16 * d + 4 * g) = v;
   }
-  // queries that met an infinite or NaN value, or an overflow between parts,
-  // again in plain fp32 (a layer of 4 x 375 frames, 8 heads of 128: 199 us, 230
+  // queries that met an infinite or NaN value, an overflow between parts or
+  // values too small for them, again in plain fp32 (a layer of 4 x 375 frames, 8 heads of 128: 199 us, 230
   // with three items half padding of NaNs, 333 with a frame of infinities that
   // every query of an item sees)
   uint64_t redo = __ballot(odd && qi < p.T);

@@ -180,3 +180,29 @@ def test_time_of_frames_that_are_not_finite():
     infinite[1, 3] = float("inf")
     assert best(padded) < 4 * plain
     assert best(infinite) < 4 * plain
+
+
+def test_tiny_values():
+    """Values too small for three bf16 parts (under 2^-110), in all heads of an
+    item and in one head of another, keep the relative error of ordinary ones;
+    items beside them are what they are without. Outputs get the size of a
+    head's values through a linear_out that scales by 2^20."""
+    d, h, B, T = 512, 8, 16, 100
+    rng = np.random.default_rng(1)
+    w = W.make_layer_weights(rng, d, h, False, False)
+    w["linear_v.weight"][:64] *= np.float32(2.0 ** -116)
+    w["linear_out.weight"] = np.eye(d, dtype=np.float32) * np.float32(2.0 ** 20)
+    layer = M.RelPositionMultiHeadAttention(d, h, False)
+    layer.load_weights(W.prefixed(w, "l"), "l")
+    layer.set_dtype(O.F32)
+    p, pos = oracle_params(w, d, h), O.RelPositionalEncoding(d, 5000, True).get_encoding(T)
+    x = rng.standard_normal((B, T, d)).astype(np.float32)
+    x[2] *= np.float32(2.0 ** -118)
+    got = forward(layer, x, pos, None, [T] * B, T)
+    for b in (0, 2, 3):
+        ref = O.mhsa_forward(p, x[b:b + 1], pos, None, None, O.F32)
+        for lo, hi in ((0, 64), (64, d)):
+            if b == 2 and lo == 0:
+                continue  # (2^-234: zeros)
+            err = np.linalg.norm(got[b:b + 1, :, lo:hi] - ref[..., lo:hi]) / np.linalg.norm(ref[..., lo:hi])
+            assert err < 2.0 ** -19, (b, lo, err)
