@@ -1418,10 +1418,10 @@ hipError_t launch(const AttnParams& p, int nb, hipStream_t s) {
 }
 
 // Key split: 16 queries per workgroup, NW waves over its key tiles.
-template <typename T, int DK, int NW>
+template <typename T, int DK, int NW, bool DEBUG>
 hipError_t launch_ks(const AttnParams& p, int nb, hipStream_t s) {
   dim3 grid((p.T + 15) / 16, p.H, nb);
-  hipLaunchKernelGGL((attn_kernel<T, DK, NW, false, true>), grid, dim3(64 * NW), 0, s, p);
+  hipLaunchKernelGGL((attn_kernel<T, DK, NW, DEBUG, true>), grid, dim3(64 * NW), 0, s, p);
   count_form(kFormKeySplit);
   return hipGetLastError();
 }
@@ -1440,10 +1440,11 @@ hipError_t dispatch_nw(const AttnParams& p, int nb, hipStream_t s) {
   // mask ran, while the key-split form of the same source is exact on those
   // shapes, so there is no one-wave form.
   if constexpr (sizeof(T) == 4) {
-    if (!dbg && (p.T <= 16 || (int64_t)nb * p.H * ((p.T + 63) / 64) <= 64))
-      return launch_ks<T, DK, 4>(p, nb, s);  // (per-wave tiles: 34 / 37 KB of LDS)
-    if (dbg) return launch<T, DK, 4, true>(p, nb, s);
-    hipLaunchKernelGGL((attn_f32_kernel<DK>), dim3(p.H, (p.T + 63) / 64, nb), dim3(256), 0, s, p);
+    if (p.T <= 16 || (int64_t)nb * p.H * ((p.T + 63) / 64) <= 64)  // (per-wave tiles: 34 / 37 KB of LDS)
+      return dbg ? launch_ks<T, DK, 4, true>(p, nb, s) : launch_ks<T, DK, 4, false>(p, nb, s);
+    const dim3 grid(p.H, (p.T + 63) / 64, nb);
+    if (dbg) hipLaunchKernelGGL((attn_f32_kernel<DK, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((attn_f32_kernel<DK, false>), grid, dim3(256), 0, s, p);
     count_form(kFormGeneric);
     return hipGetLastError();
   } else {

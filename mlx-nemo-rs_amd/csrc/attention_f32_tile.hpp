@@ -116,7 +116,8 @@ __device__ __forceinline__ void attn_f32_plain(const AttnParams& p, int bl, int 
   for (int n = 0; n < N; ++n) orow[64 * n] = nan ? NAN : o[n] * inv;
 }
 
-template <int DK>
+// DEBUG: the position scores of the tiles it walks also go to dbg_bd.
+template <int DK, bool DEBUG>
 __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const AttnParams p) {
   using C = F32Attn<DK>;
   constexpr int NKF = DK / 32, ND = DK / 16, NK = C::NK, QB = C::QB;
@@ -336,7 +337,10 @@ __global__ __launch_bounds__(256, F32Attn<DK>::WPS) void attn_f32_kernel(const A
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int u = e >> 2, r = e & 3, jl = 16 * u + 4 * g + r;
-      const float v = (sh[u][r] + sl[u][r]) * sc_qk + Rm[ql * C::RMP + jl + 15 - ql] * sc_bd;
+      const float bd = Rm[ql * C::RMP + jl + 15 - ql];
+      if (DEBUG && qi < p.T && j0 + jl < p.L)
+        p.dbg_bd[(((int64_t)b * p.H + h) * p.T + qi) * p.L + j0 + jl] = p.scale_bd * bd;
+      const float v = (sh[u][r] + sl[u][r]) * sc_qk + bd * sc_bd;
       sc[e] = full || in_interval(j0 + jl, iv) ? v : -INFINITY;
       tmax = fmaxf(tmax, sc[e]);
     }

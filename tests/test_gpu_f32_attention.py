@@ -206,3 +206,29 @@ def test_tiny_values():
                 continue  # (2^-234: zeros)
             err = np.linalg.norm(got[b:b + 1, :, lo:hi] - ref[..., lo:hi]) / np.linalg.norm(ref[..., lo:hi])
             assert err < 2.0 ** -19, (b, lo, err)
+
+
+# long inputs (the ring of position blocks turns several times) and short ones
+@pytest.mark.parametrize("d,h,B,T,form", [(512, 8, 8, 230, "generic"), (256, 2, 32, 161, "generic"),
+                                          (1024, 8, 4, 353, "generic"), (512, 8, 2, 129, "generic_key_split"),
+                                          (256, 2, 1, 97, "generic_key_split")])
+def test_position_scores_of_the_kernel_that_runs(d, h, B, T, form):
+    """The position scores that the debug entry gives are those of the kernel
+    that a forward of this shape runs, and match the rel_shift of (q + v) P^T
+    over the kernel's own q and P: products of d_k terms in fp32, rounded d_k
+    times at most, once when a sum's halves meet and once when scaled."""
+    rng, layer, p, pos = make(d, h, T, d + T)
+    x = torch.from_numpy(rng.standard_normal((B, T, d)).astype(np.float32)).cuda()
+    pos = torch.from_numpy(pos).float().cuda().contiguous()
+    before = M.debug_attention_forms()
+    got, q, P = layer.debug_position_scores(x, pos, with_inputs=True)
+    after = M.debug_attention_forms()
+    assert {k for k in after if after[k] > before[k]} == {form}
+    dk = d // h
+    q = q.cpu().numpy().astype(np.float64).reshape(B, T, h, dk).transpose(0, 2, 1, 3)
+    P = P.cpu().numpy().astype(np.float64).reshape(2 * T - 1, h, dk).transpose(1, 2, 0)
+    qv = (q.astype(np.float32) + np.float32(p.pos_bias_v).reshape(1, h, 1, dk)).astype(np.float64)
+    scale = O.f32_scale(dk)
+    ref = scale * O.rel_shift(np.matmul(qv, P[None]))[..., :T]
+    mag = scale * O.rel_shift(np.matmul(np.abs(qv), np.abs(P[None])))[..., :T]
+    assert (np.abs(got.cpu().numpy() - ref) <= (dk + 2) * 2.0 ** -24 * mag).all()
