@@ -781,11 +781,11 @@ hipError_t launch_f32_tile(const GemmParams& p, int splits, hipStream_t s) {
 //
 // Tile: the large one (64 x 128 for bf16 weights, 64 x 64 else) from 512
 // tiles, two per CU, on; 32 x 64 below (1500 x 4096 x 1024: bf16 44 / 54,
-// fp32 85 / 102, u8 88 / 109 us; 1500 x 1024 x 1024: bf16 18.2 / 15.5, fp32
-// 28.3 / 27.4, u8 28.8 / 27.9; 450 x 4096 fp32 30 / 34).
+// fp32 118 / 126, u8 103 / 112 us; 1500 x 1024 x 1024: bf16 18.2 / 15.5, fp32
+// 33.8 / 30.0, u8 33.9 / 30.4; 450 x 4096 fp32 36.5 / 37.9).
 // A contraction past 1024 is split while the tiles stay under three per CU
-// (K = 4096, N = 1024, fp32 weights: 14 rows 32 -> 10.6 in eight, 224 rows
-// 35 -> 22.6 in four, 700 rows 59 -> 48 in two, the sum pass included).
+// (K = 4096, N = 1024, fp32 weights: 14 rows 35 -> 12.5 in eight, 224 rows
+// 37.5 -> 25.2 in four, 700 rows 62.5 -> 56.5 in two, the sum pass included).
 template <int WK>
 bool takes_kpar(const GemmParams& p) {
   if (!kpar_ok<float>(p)) return false;

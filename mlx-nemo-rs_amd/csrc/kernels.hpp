@@ -64,8 +64,8 @@ struct GemmParams {
   float res_scale = 1.f;
 };
 constexpr int kActSilu = 1;
-// Scratch the K-split path can use: 64x64 tiles x splits stays <= ~512
-// workgroups, so M*N*splits <= kGemmPartialElems.
+// Scratch the K-split paths can use, M*N*splits floats: 64x64 tiles x splits up
+// to ~512 workgroups, the fp32 tiles' 32x64 ones up to 768.
 constexpr int64_t kGemmPartialElems = (int64_t)1 << 22;
 hipError_t gemm(DType dt, bool quantized, const GemmParams& p, hipStream_t s);
 // gemm()'s argument checks alone (p.M > 0 assumed).
@@ -84,7 +84,7 @@ bool gemm_tile_form(DType dt, bool quantized, const GemmParams& p, TileForm& f);
 // is launched.
 bool gemm_pair_ok(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2);
 hipError_t gemm_pair(DType dt, bool quantized, const GemmParams& p1, const GemmParams& p2, hipStream_t s);
-// Whether gemm() takes this problem with C2 / acopy set (fp32, few rows).
+// Whether gemm() takes this problem with C2 / acopy set (fp32).
 bool gemm_split_fused_ok(DType dt, const GemmParams& p);
 // Compute units of the current device (256 if the query fails), read once
 // per device.

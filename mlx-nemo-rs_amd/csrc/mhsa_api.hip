@@ -1156,7 +1156,7 @@ int32_t stream_step(mhsa_layer* L, mhsa_stream* S, const void* x, int B, int T, 
   } else {
     // One launch when the layer holds the stacked [3D, D] weight: Q to `q`,
     // K|V to the cache ring's rows of this chunk, and the chunk's input rows
-    // copied into the input ring by the workgroups of the first column tile.
+    // copied into the input ring.
     if (one_launch) {
       for (int r = ps_kv.reps(); r > 0; --r) HIPCHK(mhsa::gemm(mhsa::kF32, L->sdev[0].quantized, fp, s));
     } else {

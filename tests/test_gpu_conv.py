@@ -167,12 +167,28 @@ def test_conv_cache_needs_causal_module():
 
 
 @pytest.mark.parametrize("dtype", [O.F32, O.BF16])
+@pytest.mark.parametrize("k,causal", [(31, False), (32, True), (33, False), (33, True), (65, False), (128, True)])
+@pytest.mark.parametrize("B,T", [(1, 15), (2, 64), (1, 130)])
+def test_long_kernels_against_oracle(dtype, k, causal, B, T):
+    """Kernels on both sides of the taps that LDS holds (32), inputs shorter
+    than the kernel and of several frame tiles."""
+    d = 256
+    rng = np.random.default_rng(k + T)
+    w = conv_weights(rng, d, k, "batch_norm", False)
+    m = _module(w, d, k, "batch_norm", causal, dtype)
+    x = _input(rng, (B, T, d), dtype)
+    lengths = [T, T - 7][:B]
+    ref, _ = O.conv_module(conv_oracle(w, "batch_norm", causal), x, dtype, lengths=lengths)
+    assert row_rel_err(host(m.forward(dev(x, dtype), lengths)), ref) < (BF16_TOL if dtype == O.BF16 else F32_TOL)
+
+
+@pytest.mark.parametrize("dtype", [O.F32, O.BF16])
 @pytest.mark.parametrize("kernel,causal", [(9, False), (9, True), (31, False), (32, True), (33, False)])
 @pytest.mark.parametrize("B,T", [(1, 1), (1, 15), (1, 17), (3, 63), (2, 65)])
 def test_frame_tiles_agree(dtype, kernel, causal, B, T):
     """An item alone or among few takes 16-frame tiles, among enough others
-    64-frame ones: the same values bit for bit, for kernels on both sides of
-    the taps that LDS holds."""
+    64-frame ones: the same values bit for bit. (Past the taps that LDS holds,
+    kernel 33, all tiles are of 64 frames.)"""
     d, many = 512, 64
     rng = np.random.default_rng(kernel + B + T)
     m = M.ConvolutionModule(d, kernel, "batch_norm", causal, True)

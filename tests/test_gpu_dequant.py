@@ -2,8 +2,9 @@
 
 The quantized projections never materialise a dequantised weight: each GEMM
 unpacks the u8 codes and applies W = s * q + b in registers, one form per
-kernel (the bf16 tile kernel in all its tile shapes, the paired Q/K/V +
-position launch, the fp32 K-parallel, tile and split kernels). Feeding unit
+kernel (the bf16 tile kernel in all its tile shapes, the bf16 kernels of few
+tiles, the paired Q/K/V + position launch, the fp32 K-parallel and tile
+kernels). Feeding unit
 rows through a kernel reads those weights back: with row r of the input equal
 to e_{r mod K}, output row r is column r mod K of W (one product 1 * w, the
 other terms exactly 0), so every output element is one dequantised weight
@@ -86,9 +87,10 @@ def gpu_layer(w, d, h, dtype):
     return layer
 
 
-# bf16 tile kernel forms at N = K = 1024: 64x64 (1024 rows), 128x128 with four
+# bf16 kernel forms at N = K = 1024: few tiles as 32x32 (200 rows), 64x32 (400)
+# and 64x64 (1024), then the tile kernel as 64x64 (1100), 128x128 with four
 # stages (2048), 192x128 (6000), 128x128 with two stages (6200), 256x256 (15000)
-@pytest.mark.parametrize("rows", [1024, 2048, 6000, 6200, 15000])
+@pytest.mark.parametrize("rows", [200, 400, 1024, 1100, 2048, 6000, 6200, 15000])
 def test_projection_dequant_bf16_tile_forms(rows):
     rng = np.random.default_rng(rows)
     w = quant_layer(rng)
@@ -98,9 +100,9 @@ def test_projection_dequant_bf16_tile_forms(rows):
         exact(layer.debug_linear(name, x), expect(deq(w, name, O.BF16), rows), f"{name} rows={rows}")
 
 
-# fp32 kernels: K-parallel with 16x16 (100 rows) and 32x32 tiles (1024), the
-# 128x128 tile kernel (6200)
-@pytest.mark.parametrize("rows", [100, 1024, 6200])
+# fp32 kernels: K-parallel with 16x16 (100 rows) and 32x32 tiles (190), the tile
+# kernel with 32x64 (1024) and 64x64 tiles (6200)
+@pytest.mark.parametrize("rows", [100, 190, 1024, 6200])
 def test_projection_dequant_f32_kernels(rows):
     rng = np.random.default_rng(100 + rows)
     w = quant_layer(rng)

@@ -901,10 +901,11 @@ def test_streaming_equals_offline_last_rows():
                                                   (512, 8, "dense")])
 def test_streaming_projection_kinds_with_biases(d_model, n_heads, kind, dtype):
     """Cache-aware steps with q/k/v/out biases and u8, dense or mixed q/k/v.
-    Same-kind q/k/v with D <= 1024 take one launch for the chunk's Q, its K|V
-    rows of the cache ring and its copy into the input ring; mixed kinds and
-    D = 1280 take separate launches. Four steps against the oracle (fp32
-    bound) and the exported cache bit-equal to the oracle's."""
+    Same-kind q/k/v take one launch for the chunk's Q, its K|V rows of the
+    cache ring and its copy into the input ring (the K-parallel kernel up to
+    D = 1024, the fp32 tiles at D = 1280); mixed kinds take separate launches.
+    Four steps against the oracle (fp32 bound) and the exported cache bit-equal
+    to the oracle's."""
     rng = np.random.default_rng(51)
     quant = kind != "dense"
     w = W.make_layer_weights(rng, d_model, n_heads, True, quant, centred=True)
