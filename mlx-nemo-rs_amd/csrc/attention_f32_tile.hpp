@@ -24,12 +24,13 @@
 // the probabilities. Rows' 16-byte chunks are XOR-permuted by the row so that
 // 16 rows of one fragment read cover all banks (V^T: an 80-byte pitch). The
 // grid has the heads first, so a head's blocks share an XCD's L2.
-// Measured, 4 x 375 frames, 8 heads of 128: 84.7 -> 56.4 us; a whole layer of
-// 3 x 1500 frames 1310 -> 830 us, of 2 x 750 frames at 8 heads of 64 146 ->
-// 108; error against 64 bits 1.0e-6 -> 3.6e-7 (4 x 375), 5.2e-7 (3 x 1500).
+// Measured, 4 x 375 frames, 8 heads of 128: 84.7 -> 61 us; a whole layer of 3 x
+// 1500 frames 1305 -> 950 us, of 2 x 750 frames at 8 heads of 64 148 -> 120;
+// error against 64 bits 9.8e-7 -> 3.6e-7 (4 x 375), 1.0e-6 -> 5.2e-7 (3 x 1500).
 // What bounds it now at d_k = 128: LDS holds one workgroup per CU, so a SIMD
-// has one wave, whose products (2,700 cycles a tile), splits and softmax
-// (some 3,500) and LDS reads add up instead of overlapping.
+// has one wave, whose 224 products (3,600 cycles a tile), vector instructions
+// (4.8 per product by the counters, 4,300 cycles) and LDS reads add up instead
+// of overlapping.
 template <int DK>
 struct F32Attn {
   static constexpr int NT = 256, QB = 64, NK = 32;

@@ -685,12 +685,12 @@ hipError_t launch_kw(const GemmParams& p, hipStream_t s) {
 // the tile kernel's. Measured, us a launch, 64 x 64 tile kernel / this:
 //   32 x 32  bf16   1 x 4096 x 1024   6.2 / 5.5,  203 x 1024 x 4096  14.7 / 9.0
 //            u8   203 x 1024 x 4096  23.9 / 12.0, 400 x 512 x 2048   14.1 / 8.2
-//   64 x 32  bf16 400 x 1024 x 4096  15.9 / 11.6, 125 x 4096 x 1024   7.6 / 7.4
+//   64 x 32  bf16 400 x 1024 x 4096  15.9 / 11.6, 700 x 512 x 2048    9.2 / 8.2
 //            u8   400 x 1024 x 4096  24.5 / 13.7, 125 x 4096 x 1024  10.3 / 7.6
 //   64 x 64  u8   700 x 1024 x 4096  25.1 / 19.6, 203 x 4096 x 1024  11.4 / 10.3
-// One dense problem does not take the 64 x 64 form (the tile kernel's four
-// waves are as fast where nothing is dequantised), but a pair does: it saves a
-// launch of 4 us.
+// One dense problem does not take the 64 x 64 form, nor 64 x 32 up to K = 1024
+// (the tile kernel's four waves are as fast where nothing is dequantised: 257 x
+// 1024 x 1024 5.8 / 6.8), but a pair does: it saves a launch of 4 us.
 template <bool QUANT>
 int chain_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
   const int64_t cus = device_cus();
@@ -698,7 +698,8 @@ int chain_form(const GemmParams& p1, const GemmParams* p2 = nullptr) {
     if (p && (!tile_ok(*p) || p->N % 64 || m_tiles<64>(*p) * (p->N / 64) < 16)) return 0;
   auto tiles = [&](auto count) { return count(p1) + (p2 ? count(*p2) : 0); };
   if (tiles([](const GemmParams& p) { return m_tiles<32>(p) * (p.N / 32); }) <= cus) return 1;
-  if (tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 32); }) <= cus) return 2;
+  if ((QUANT || p2 || p1.K > 1024) && tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 32); }) <= cus)
+    return 2;
   if ((QUANT || p2) && tiles([](const GemmParams& p) { return m_tiles<64>(p) * (p.N / 64); }) <= cus) return 3;
   return 0;
 }

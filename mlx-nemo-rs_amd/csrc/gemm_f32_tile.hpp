@@ -134,9 +134,11 @@ __device__ __forceinline__ void f32_store(const GemmParams& p, bool ok, int row,
 // stream raw through NS LDS stages of 64 k-columns with direct-to-LDS loads
 // (fp32 rows are 4 bytes a value there against 6 for their parts), and each
 // wave splits its fragments in registers, one step ahead, between the MFMAs
-// of the step before. The vector work is what bounds it now: a wave has room
-// for 6 vector instructions per MFMA beside another wave's (measured), and
-// the split of a fragment takes 44, so the waves share a tile along K first,
+// of the step before. The vector work is what bounds it now: the counters show
+// 8 to 11 vector instructions per MFMA (the 64 x 64 and 32 x 64 tiles of fp32
+// weights; 7.6 in the 64 x 128 ones of bf16 weights), whose 32 cycles hold 8,
+// and MFMAs a third of the time (profiles/mfma_utilization.txt). The split of a
+// fragment takes 44, so the waves share a tile along K first,
 // where no fragment is split twice, and along M only with bf16 weights, which
 // need no split; two workgroups per CU overlap each other's barriers.
 // Measured (us before / now, MFMA rate now in bf16 products), 1500 rows:
