@@ -65,7 +65,8 @@ def test_linears(d, f, rows, quant):
 
 
 # K of 1 to 64 stages (phases of four or two, ends inside one), and every tile
-# form: 32 x 32 up to 256 rows of 1024 columns, 64 x 32 up to 512, 64 x 64
+# form: 32 x 32 up to 256 rows of 1024 columns, 64 x 32 up to 512 (u8, and
+# dense past K = 1024), 64 x 64 (u8; dense ones take the tile kernel)
 @pytest.mark.parametrize("quant", [False, True])
 @pytest.mark.parametrize("k,rows", [(64, 40), (128, 33), (192, 1), (256, 64), (320, 31), (384, 257), (448, 65), (512, 500),
                                     (576, 129), (704, 400), (1024, 203), (1024, 700), (1344, 300), (2240, 97),
